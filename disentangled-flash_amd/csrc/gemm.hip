@@ -14,34 +14,57 @@
 //                  of DebertaV2SelfOutput / DebertaV2Output before LayerNorm,
 //                  _reference.py:108-112, 482-485)
 //
-// Tiling.  A workgroup of WAVES_M x WAVES_N wavefronts computes a 256 x BN
-// tile of Y (GemmConfig below: 256 x 192 with 4 or 8 wavefronts, 256 x 128
-// with 4 wavefronts at two workgroups per CU).  K is walked in steps of 32
-// through a ring of LDS stages.  Global -> LDS copies use
-// global_load_lds_dwordx4: no registers, no VALU; each instruction of a
-// wavefront writes 1 KB of LDS in lane order, so the LDS layout is chosen by
-// which global chunk each lane fetches.  Rows of the K-step are 64 bytes; two
-// rows form a 128-byte line, and the eight 16-byte chunks of a line are
-// XOR-swizzled with the line index, which makes the MFMA fragment reads
-// (ds_read_b128, 16 rows x one k-slice per 16 lanes) bank-conflict free.
+// What bounds it.  With tiles of 256 rows the k-loop is near the matrix unit:
+// at M = 16384, N = K = 3072 (fp16) the 256 x 256 tile takes 235 us, 1.32
+// PFLOP/s, its matrix pipe busy 66-70 % at the clock the power limit leaves
+// (1.8 GHz); a loop of 32-deep steps in the compiler's own order took 292 us.  At
+// K = 768 the rest is the start of a tile and the stores at its end (16384 rows:
+// QKV 62 us, 920 TFLOP/s; FFN intermediate with GELU 85-90 us); with few rows it is the
+// latency of the copies.
+
+// Slabs of 64 k.  X and W are copied straight into LDS (buffer loads with the
+// LDS bit, 16 bytes a lane: no registers, no address arithmetic in the loop)
+// as slabs of 64 k, so that a row of a copy is one whole 128-byte line: with
+// 32-deep slabs (64-byte rows) L2 serves twice as many requests for the same
+// bytes (256 x 256 tile, N = K = 3072: 250 against 235 us).  A slab row is 128 bytes of LDS whose
+// eight 16-byte chunks are permuted by slab_swizzle(row), which makes the
+// MFMA fragment reads (16 rows x one chunk per 16 lanes) conflict-free.  STAGES
+// slabs form a ring.
 //
-// MFMA v_mfma_f32_16x16x32_{f16,bf16} with the weight as the A operand and the
-// activation as B, so the accumulator of lane (c, g) holds Y[m0 + c][n0 + 4g ..
-// n0 + 4g + 3]: four consecutive outputs of one row.  The epilogue stages the
-// tile through LDS and writes it in coalesced 16-byte chunks.
+// One slab is two 32-deep MFMA steps.  The fragments of a step are read from
+// LDS during the MFMAs of the step before (two register sets).  Between the
+// two steps of slab t stands the only barrier of the slab: every wavefront has
+// then its last fragments of slab t in registers and its own copies of slab
+// t + 1 have landed, so that after it slab t + 1 may be read and slab t be
+// overwritten by the copies of slab t + STAGES, which are issued during the
+// second step.
 //
-// Launch order: workgroup p runs on XCD p % 8.  Each XCD takes a contiguous
-// range of tiles.  When X is the larger operand (M >= N: many rows) the range
-// is row-major (column blocks fastest), so the tiles of one X row block run on
-// the same XCD and share its L2, and every XCD streams all of W; when W is the
-// larger (few rows) it is column-major, so every XCD streams all of X and only
-// its own slice of W (at 512 rows this takes the 1536-wide QKV from 26.2 to
-// 17.9 us and the FFN intermediate from 28.0 to 21.6 us, bf16).
+// The order inside a step is written down (sched_barrier between the groups):
+// fragment reads and copies are spread over the first three quarters of the
+// MFMAs.  Left to the compiler they all come first, and the matrix pipe waits
+// for them: 255 against 235 us (N = K = 3072), 82 against 78.5 us at K = 768.
+//
+// MFMA v_mfma_f32_16x16x32_{f16,bf16} with the weight as the A operand, so a
+// lane's accumulators of a 16 x 16 block are four consecutive outputs of one
+// row.  The rows of W are assigned to the blocks so that the blocks 2i and
+// 2i + 1 of a lane hold eight consecutive outputs (w_row): the epilogue writes
+// 16 bytes a lane straight from the registers, with no pass through LDS.
+//
+// Launch order: workgroup p runs on XCD p % 8.  The tiles are split over the XCDs
+// in a grid of xcds_m x 8 / xcds_m ranges, so that the rows of X and of W that one
+// XCD reads, which its L2 keeps, are few (launch_gemm; 2048 x 4608 x 1536 on
+// 128 x 192 tiles 40 -> 33 us against ranges of whole rows).
+//
+// k order: every XCD starts at a slab of its own and wraps around.  All tiles walk
+// k together, and rows are K * 2 bytes apart, so with K = 3072 or 6144 the rows of
+// one slab lie in a few of the memory channels only; eight starting points reach
+// eight times as many (4096 x 768 x 3072 30.4 -> 25.4 us, 2048 x 1536 x 6144 57 -> 53).
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "device_common.h"
 #include "dflash.h"
@@ -50,66 +73,77 @@ namespace dflash {
 
 namespace {
 
-typedef __attribute__((address_space(3))) void lds_void_t;
-
-constexpr int kGemmThreads = 256;  // 4 wavefronts, 2 x 2 over the tile
-constexpr int kBK = 32;            // K per stage (one MFMA k-step)
+constexpr int kStepK = 32;           // k of one MFMA step
+constexpr int kSlabK = 2 * kStepK;    // k of one slab (128-byte rows)
 
 constexpr int kEpiBias = 0;
 constexpr int kEpiBiasGelu = 1;
 constexpr int kEpiBiasAdd = 2;
 
-// Byte offset inside a stage's X or W tile of (row, 16-byte chunk c in 0..3).
-// Two 64-byte rows form line row/2; chunk position p = 4*(row&1) + c is
-// XOR-swizzled with the line index.
-__device__ constexpr int swz_offset(int row, int c) {
-  const int line = row >> 1;
-  const int p = ((row & 1) << 2) | c;
-  return line * 128 + ((p ^ (line & 7)) << 4);
+// Chunk permutation of slab row r: 16-byte chunk k of the row sits at position
+// k ^ slab_swizzle(r).  Eight consecutive rows hit eight different chunks of a
+// 128-byte window, and of sixteen no two the same chunk of a 256-byte one.
+// Depends on r mod 16 only.
+__device__ constexpr int slab_swizzle(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+// Output column (inside the tile) of W row r of a slab: row x = 4a + b of the
+// 16-row blocks 2i and 2i + 1 holds columns 32i + 8a + b and 32i + 8a + 4 + b.
+__device__ constexpr int w_row(int r) {
+  const int block = r >> 4;
+  const int x = r & 15;
+  return 8 * (x >> 2) + (x & 3) + 4 * (block & 1) + 32 * (block >> 1);
 }
 
-// The inverse for the copy: LDS slot s (16 bytes, lane order) -> (row, chunk).
-__device__ inline void swz_slot(int s, int& row, int& c) {
-  const int line = s >> 3;
-  const int p = (s & 7) ^ (line & 7);
-  row = 2 * line + (p >> 2);
-  c = p & 3;
-}
-
-// GELU in its erf form, 0.5 x (1 + erf(x / sqrt 2)), with erf from
-// Abramowitz & Stegun, Handbook of Mathematical Functions, formula 7.1.26:
-//   erf(z) = 1 - (a1 t + a2 t^2 + a3 t^3 + a4 t^4 + a5 t^5) exp(-z^2),
-//   t = 1 / (1 + p z), z >= 0, |error| <= 1.5e-7.
-// For x < 0 the complement 1 + erf(-|z|) = (a1 t + ...) exp(-z^2) is used
-// directly, so the small values of the negative tail carry no cancellation.
-// About 12 instructions against ~40 for the library erff with both of its
-// branches; the difference is far below the fp16/bf16 rounding of the output.
+// GELU in its erf form, x Phi(x), with Phi(-a) = 2^P(a) for a = |x|: P is a
+// polynomial of degree 8 fitted to log2 Phi(-a) on [0, 6] (minimax weighted with
+// the error it makes in x Phi(x); its leading coefficient is held negative, so P
+// falls without bound past the range and 2^P goes to 0).  Evaluated in fp32 the
+// result is within 3.8e-7 of the exact value over all fp16 and bf16 inputs, and
+// the negative tail carries no cancellation; 49 fp16 inputs round to another
+// value than the exact result does, 257 with formula 7.1.26 of Abramowitz & Stegun,
+// which it replaced and which needed a reciprocal besides the exponential and
+// about a quarter more issue slots.
 __device__ inline float gelu_erf(float x) {
-  constexpr float kP = 0.3275911f;
-  constexpr float kA1 = 0.254829592f, kA2 = -0.284496736f, kA3 = 1.421413741f,
-                  kA4 = -1.453152027f, kA5 = 1.061405429f;
-  const float z = fabsf(x) * 0.70710678118654752440f;
-  const float t = __builtin_amdgcn_rcpf(fmaf(kP, z, 1.0f));
-  const float poly = t * fmaf(t, fmaf(t, fmaf(t, fmaf(t, kA5, kA4), kA3), kA2), kA1);
-  const float tail = poly * __builtin_amdgcn_exp2f(-z * z * 1.44269504088896341f);  // erfc(z)
-  const float phi = x >= 0.0f ? 1.0f - 0.5f * tail : 0.5f * tail;                // Phi(x)
-  return x * phi;
+  constexpr float kP[9] = {-0.9999997615814209f,   -1.1511133909225464f,
+                           -0.459148645401001f,    -0.05266685038805008f,
+                           0.007304247934371233f,  -0.0003195464378222823f,
+                           -0.00011073797941207886f, 2.3465026970370673e-05f,
+                           -1.500000053056283e-06f};
+  const float a = fabsf(x);
+  float p = kP[8];
+#pragma unroll
+  for (int k = 7; k >= 0; --k) p = fmaf(p, a, kP[k]);
+  const float tail = __builtin_amdgcn_exp2f(p);  // Phi(-|x|)
+  return x * (x >= 0.0f ? 1.0f - tail : tail);
 }
 
-// One global_load_lds_dwordx4: 16 bytes from `src` (per lane) to LDS at
-// `lds_base` + 16 * lane (`lds_base` wavefront-uniform).  Kept in a __device__
-// function: used directly inside the kernel body, the builtin stops clang's host
-// pass from emitting the kernel's launch stub.
-__device__ inline void copy16_to_lds(const void* src, unsigned char* lds_base) {
-  __builtin_amdgcn_global_load_lds(src, (lds_void_t*)lds_base, 16, 0, 0);
+// One buffer_load_dwordx4 with the LDS bit: 16 bytes per lane from `off` + `koff`
+// (`koff` uniform and not range-checked; rows past the tile's last have `off` past
+// the resource's size and store zeros) to LDS at `lds` + 16 * lane (`lds` uniform,
+// in M0; one wait state between the write of M0 and the load).  Inline assembly,
+// so that the compiler does not wait for copies in flight before fragment reads;
+// they are awaited by wait_vmem and the slab's barrier.
+__device__ inline void copy16_to_lds(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t koff,
+                                     uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %1, %2, %3 offen lds"
+      :
+      : "s"(lds), "v"(off), "s"(r), "s"(koff)
+      : "memory");
 }
 
-// s_barrier after this wavefront's LDS reads have returned, without the memory
-// fence of __syncthreads() (which would wait for every pending copy and drain
-// the pipeline).  The copies' LDS writes are published by the explicit vmcnt
-// waits before it; the memory clobber keeps LDS accesses on their side.
-__device__ inline void workgroup_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+// The same from a 64-bit address per lane, for operands whose tile does not fit
+// the 32-bit offsets of a buffer resource.
+__device__ inline void copy16_to_lds_far(const void* src, uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off"
+      :
+      : "s"(lds), "v"(src)
+      : "memory");
 }
 
 // Wait until at most N of this thread's vector-memory operations are pending.
@@ -123,44 +157,31 @@ __device__ inline void wait_vmem() {
 
 // Tile configuration: a workgroup of WAVES_M x WAVES_N wavefronts computes a
 // BM x BN tile of Y (wavefront tile BM/WAVES_M x BN/WAVES_N) through a ring of
-// STAGES LDS stages; WGS workgroups per CU are budgeted for.
-template <int BN_, int STAGES_, int WGS_, int WAVES_M_, int WAVES_N_, int BM_ = 256>
+// STAGES slabs; WGS workgroups per CU are budgeted for.
+template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int WGS_, int STAGES_ = 2>
 struct GemmConfig {
   static constexpr int BM = BM_;
   static constexpr int BN = BN_;
-  static constexpr int STAGES = STAGES_;
-  static constexpr int WGS = WGS_;
   static constexpr int WAVES_M = WAVES_M_;
   static constexpr int WAVES_N = WAVES_N_;
-  static constexpr int THREADS = 64 * WAVES_M * WAVES_N;
+  static constexpr int WGS = WGS_;
+  static constexpr int STAGES = STAGES_;
+  static constexpr int WAVES = WAVES_M * WAVES_N;
+  static constexpr int THREADS = 64 * WAVES;
   static constexpr int WM = BM / WAVES_M;
   static constexpr int WN = BN / WAVES_N;
-  static constexpr int MB = WM / 16;                 // 16-row blocks per wavefront
-  static constexpr int NB = WN / 16;                 // 16-column blocks per wavefront
-  static constexpr int A_CHUNKS = BM * kBK / 8;      // 16-byte chunks of a stage's X tile
-  static constexpr int B_CHUNKS = BN * kBK / 8;
-  // Copy instructions per thread per stage.  A chunk count that is not a
-  // multiple of the workgroup size leaves the last round to the first
-  // wavefronts (whole wavefronts, so the counts stay wavefront-uniform).
-  static constexpr int A_LOADS = (A_CHUNKS + THREADS - 1) / THREADS;
-  static constexpr int B_LOADS = (B_CHUNKS + THREADS - 1) / THREADS;
-  static constexpr int A_BYTES = BM * kBK * 2;
-  static constexpr int STAGE_BYTES = (BM + BN) * kBK * 2;
-  static constexpr int TILE_LD = BN + 8;             // epilogue staging row (elements)
-  static constexpr int RING = STAGES * STAGE_BYTES;
-  static constexpr int STAGING = BM * TILE_LD * 2;
-  static constexpr int LDS = RING > STAGING ? RING : STAGING;
-  static_assert(A_CHUNKS % 64 == 0 && B_CHUNKS % 64 == 0, "copies in whole wavefronts");
-  static_assert(WM % 16 == 0 && WN % 16 == 0, "wavefront tile of whole MFMA blocks");
-  static_assert(STAGES >= 3, "the pipeline keeps STAGES - 2 stages in flight");
-  static_assert((STAGES - 2) * (A_LOADS + B_LOADS) <= 63, "vmcnt range");
-  // Copies a wavefront issues per stage (its last rounds may be partial).
-  __device__ static constexpr int loads_of(int wave) {
-    int n = 0;
-    for (int j = 0; j < A_LOADS; ++j) n += (j * THREADS + wave * 64 < A_CHUNKS) ? 1 : 0;
-    for (int j = 0; j < B_LOADS; ++j) n += (j * THREADS + wave * 64 < B_CHUNKS) ? 1 : 0;
-    return n;
-  }
+  static constexpr int MB = WM / 16;            // 16-row blocks per wavefront
+  static constexpr int NB = WN / 16;            // 16-column blocks per wavefront
+  static constexpr int A_LOADS = BM / 8 / WAVES;  // copies (8 rows each) per wavefront and slab
+  static constexpr int B_LOADS = BN / 8 / WAVES;
+  static constexpr int LOADS = A_LOADS + B_LOADS;
+  static constexpr int A_BYTES = BM * kSlabK * 2;
+  static constexpr int SLAB = (BM + BN) * kSlabK * 2;
+  static constexpr int LDS = STAGES * SLAB;
+  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "copies split evenly");
+  static_assert(WM % 16 == 0 && WN % 32 == 0, "whole MFMA blocks, column blocks in pairs");
+  static_assert(STAGES >= 2 && LDS * WGS <= 160 * 1024, "LDS of a CU");
+  static_assert((STAGES - 1) * LOADS <= 63, "vmcnt range");
 };
 
 struct GemmArgs {
@@ -171,17 +192,19 @@ struct GemmArgs {
   void* y;
   int M, N, K;
   int m_blocks, n_blocks;
-  int col_major;  // tile order within an XCD's range: column blocks slowest
+  int xcds_m;  // XCDs along the rows (1, 2, 4, 8); 8 / xcds_m along the columns
 };
 
-template <typename T, int EPI, typename CF>
+// FAR: 64-bit copy addresses (tile rows past 32-bit byte offsets).
+template <typename T, int EPI, typename CF, bool FAR = false>
 __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) {
   using M = Mma<T>;
   using F = typename M::frag;
-  constexpr int BN = CF::BN;
-  constexpr int S = CF::STAGES;
   constexpr int MB = CF::MB;
   constexpr int NB = CF::NB;
+  constexpr int S = CF::STAGES;
+  constexpr int kMfmas = MB * NB;   // of one step
+  constexpr int kReads = MB + NB;   // fragment reads of one step
   extern __shared__ __align__(16) unsigned char smem[];
 
   const int tid = threadIdx.x;
@@ -191,74 +214,84 @@ __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) 
   const int g = lane >> 4;
   const int wm = wave % CF::WAVES_M;  // wavefront row block
   const int wn = wave / CF::WAVES_M;  // wavefront column block
-  constexpr int NT = CF::THREADS;
 
-  // Tile of this workgroup (XCD-aware order, see the file comment).
-  const int total = a.m_blocks * a.n_blocks;
+  // Tile of this workgroup (see the file comment): the tile ranges of XCD p % 8,
+  // columns fastest.
   const int p = blockIdx.x;
-  const int per_xcd = (total + 7) >> 3;
-  const int t = (p & 7) * per_xcd + (p >> 3);
-  if (t >= total) return;  // padding of the grid to a multiple of 8
-  int mb, nb;
-  if (a.col_major) {
-    nb = t / a.m_blocks;
-    mb = t - nb * a.m_blocks;
-  } else {
-    mb = t / a.n_blocks;
-    nb = t - mb * a.n_blocks;
-  }
+  const int xm = (p & 7) % a.xcds_m;
+  const int xn = (p & 7) / a.xcds_m;
+  const int m_lo = a.m_blocks * xm / a.xcds_m;
+  const int n_lo = a.n_blocks * xn * a.xcds_m / 8;
+  const int cols = a.n_blocks * (xn + 1) * a.xcds_m / 8 - n_lo;
+  const int mt = (p >> 3) / max(cols, 1);
+  const int mb = m_lo + mt;
+  const int nb = n_lo + (p >> 3) - mt * cols;
+  if (cols == 0 || mb >= a.m_blocks * (xm + 1) / a.xcds_m) return;  // ranges differ in size
   const int m_base = mb * CF::BM;
-  const int n_base = nb * BN;
+  const int n_base = nb * CF::BN;
   const int K = a.K;
+  const int KT = (K + kSlabK - 1) / kSlabK;  // slabs (the last may be half: K is a multiple of 32)
+  const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
+  const int rows = min(CF::BM, a.M - m_base);
+  const T* X = reinterpret_cast<const T*>(a.x) + static_cast<int64_t>(m_base) * K;
+  const T* W = reinterpret_cast<const T*>(a.w) + static_cast<int64_t>(n_base) * K;
+  const uint32_t x_bytes = static_cast<uint32_t>(rows) * row_bytes;
+  const uint32_t w_bytes = static_cast<uint32_t>(CF::BN) * row_bytes;
 
-  const T* X = reinterpret_cast<const T*>(a.x);
-  const T* W = reinterpret_cast<const T*>(a.w);
-
-  // Per-thread source pointers of its copy slots (advance by kBK per stage).
-  const T* asrc[CF::A_LOADS];
-  const T* bsrc[CF::B_LOADS];
+  // Copy j of a slab fetches eight slab rows (8 lanes a row): row and source
+  // chunk of this lane, and its byte offset from the tile's first row.
+  auto slab_row = [&](int j) { return (j * CF::WAVES + wave) * 8 + (lane >> 3); };
+  auto chunk_of = [&](int r) { return (lane & 7) ^ slab_swizzle(r); };
+  uint32_t xoff[CF::A_LOADS], woff[CF::B_LOADS];
 #pragma unroll
-  for (int j = 0; j < CF::A_LOADS; ++j) {
-    int row, ch;
-    swz_slot(min(j * NT + tid, CF::A_CHUNKS - 1), row, ch);
-    const int m = min(m_base + row, a.M - 1);  // rows past M repeat row M-1 (never stored)
-    asrc[j] = X + static_cast<int64_t>(m) * K + ch * 8;
-  }
+  for (int j = 0; j < CF::A_LOADS; ++j)
+    xoff[j] = static_cast<uint32_t>(slab_row(j)) * row_bytes + chunk_of(slab_row(j)) * 16;
 #pragma unroll
-  for (int j = 0; j < CF::B_LOADS; ++j) {
-    int row, ch;
-    swz_slot(min(j * NT + tid, CF::B_CHUNKS - 1), row, ch);
-    bsrc[j] = W + static_cast<int64_t>(n_base + row) * K + ch * 8;
-  }
-  // LDS destinations: wavefront-uniform bases of each copy instruction; a
-  // wavefront whose slots of a round lie past the tile skips that round.
-  auto issue = [&](int stage, int kt) {
-    unsigned char* sa = smem + stage * CF::STAGE_BYTES;
-    unsigned char* sb = sa + CF::A_BYTES;
-    const int koff = kt * kBK;
-#pragma unroll
-    for (int j = 0; j < CF::A_LOADS; ++j)
-      if (CF::A_CHUNKS % NT == 0 || j * NT + wave * 64 < CF::A_CHUNKS)
-        copy16_to_lds(asrc[j] + koff, sa + (j * NT + wave * 64) * 16);
-#pragma unroll
-    for (int j = 0; j < CF::B_LOADS; ++j)
-      if (CF::B_CHUNKS % NT == 0 || j * NT + wave * 64 < CF::B_CHUNKS)
-        copy16_to_lds(bsrc[j] + koff, sb + (j * NT + wave * 64) * 16);
+  for (int j = 0; j < CF::B_LOADS; ++j)
+    woff[j] = static_cast<uint32_t>(w_row(slab_row(j))) * row_bytes + chunk_of(slab_row(j)) * 16;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
+  // The k order starts at a slab of its own on each XCD and wraps around.
+  const int k0 = K % kSlabK == 0 ? ((p & 7) * KT) >> 3 : 0;
+  auto slab_at = [&](int kt) { return kt + k0 < KT ? kt + k0 : kt + k0 - KT; };
+  // Copy j of slab `kt` into ring stage `stage`.  Past the last slab it fetches
+  // nothing (a resource of size 0: zeros into a stage that is not read again),
+  // so that every slab issues the same number of copies and the waits are
+  // compile-time.
+  auto copy = [&](int j, int kt, uint32_t stage) {
+    const bool is_x = j < CF::A_LOADS;
+    const int jj = is_x ? j : j - CF::A_LOADS;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(
+        lds0 + stage * CF::SLAB + (is_x ? 0 : CF::A_BYTES) + (jj * CF::WAVES + wave) * 1024);
+    if constexpr (FAR) {
+      // Rows past M repeat row M - 1; slabs and chunks past K repeat k 0 .. 31 of the
+      // last 32 (their products are not computed).
+      const int r = is_x ? min(slab_row(jj), rows - 1) : w_row(slab_row(jj));
+      const int k = min(slab_at(min(kt, KT - 1)) * kSlabK + chunk_of(slab_row(jj)) * 8, K - 8);
+      copy16_to_lds_far((is_x ? X : W) + static_cast<int64_t>(r) * K + k, dst);
+    } else {
+      const uint32_t bytes = kt < KT ? (is_x ? x_bytes : w_bytes) : 0u;
+      const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<T*>(is_x ? X : W), static_cast<short>(0), static_cast<int>(bytes), 0x00020000);
+      copy16_to_lds(rsrc, is_x ? xoff[is_x ? jj : 0] : woff[is_x ? 0 : jj],
+                    __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(slab_at(kt)) * (kSlabK * 2)), dst);
+    }
   };
 
-  // Lane-constant fragment offsets: X rows wm*WM + 16*i + c, W rows wn*WN + 16*i + c,
-  // k-slice g.  Every fragment address is a multiple of 16 bytes; saying so
-  // keeps the reads single ds_read_b128 (the library is built with unaligned
-  // LDS access off, where an unproven alignment becomes byte reads).
-  const int xoff = swz_offset(wm * CF::WM + c, g);
-  const int woff = swz_offset(wn * CF::WN + c, g);
-  auto x_frag = [&](int stage, int i) {
-    return *static_cast<const F*>(__builtin_assume_aligned(
-        smem + stage * CF::STAGE_BYTES + xoff + i * 16 * 64, 16));
+  // Fragments of step u (0, 1) of a slab at LDS byte `base`: X rows wm*WM + 16i + c,
+  // W rows wn*WN + 16i + c, chunk 4u + g.  Every address is a multiple of 16 bytes;
+  // saying so keeps the reads single ds_read_b128 (the library is built with
+  // unaligned LDS access off, where an unproven alignment becomes byte reads).
+  const int swz = slab_swizzle(c);
+  const int chunk[2] = {(g ^ swz) * 16, ((4 + g) ^ swz) * 16};
+  const int xrow = (wm * CF::WM + c) * (kSlabK * 2);
+  const int wrow = CF::A_BYTES + (wn * CF::WN + c) * (kSlabK * 2);
+  auto x_frag = [&](uint32_t base, int u, int i) {
+    return *static_cast<const F*>(
+        __builtin_assume_aligned(smem + base + xrow + chunk[u] + i * 16 * kSlabK * 2, 16));
   };
-  auto w_frag = [&](int stage, int i) {
-    return *static_cast<const F*>(__builtin_assume_aligned(
-        smem + stage * CF::STAGE_BYTES + CF::A_BYTES + woff + i * 16 * 64, 16));
+  auto w_frag = [&](uint32_t base, int u, int i) {
+    return *static_cast<const F*>(
+        __builtin_assume_aligned(smem + base + wrow + chunk[u] + i * 16 * kSlabK * 2, 16));
   };
 
   f32x4_t acc[NB][MB];
@@ -266,165 +299,121 @@ __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) 
   for (int i = 0; i < NB; ++i)
 #pragma unroll
     for (int j = 0; j < MB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  F xf[2][MB], wf[2][NB];
 
-  // Pipeline over the k-steps kt = 0 .. KT-1 with a ring of S LDS stages
-  // (k-step kt in stage kt % S).  While the MFMAs of kt run from registers, the
-  // fragments of kt + 1 are read from LDS and the copies of kt + 2 .. kt + S - 1
-  // are in flight.  One barrier per k-step: it publishes the copies of kt + 1
-  // and guarantees that every wavefront has its fragments of kt in registers,
-  // so stage kt % S is refilled with k-step kt + S right after it.  Every
-  // iteration issues one stage of copies (past the last k-step it re-fetches
-  // k-step KT - 1 into a stage nobody reads again), so the number of copies in
-  // flight is the same in every iteration and the waits are compile-time.
-  const int KT = K / kBK;
 #pragma unroll
-  for (int s0 = 0; s0 < S; ++s0) issue(s0, min(s0, KT - 1));
-  F xf[MB], wf[NB], wnext[NB];
-  // Waits: copies of k-step kt + 1 are complete once at most those of
-  // kt + 2 .. kt + S - 1 are pending.  The per-stage count of a wavefront is
-  // one of two compile-time values (full or short last copy round).
-  constexpr int kLoadsHi = CF::loads_of(0);
-  constexpr int kLoadsLo = CF::loads_of(CF::WAVES_M * CF::WAVES_N - 1);
-  const bool short_wave = CF::loads_of(wave) != kLoadsHi;
-  auto wait_next = [&]() {
-    if (short_wave) {
-      wait_vmem<(S - 2) * kLoadsLo>();
-    } else {
-      wait_vmem<(S - 2) * kLoadsHi>();
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int j = 0; j < CF::LOADS; ++j) copy(j, s, s);
+  wait_vmem<(S - 1) * CF::LOADS>();  // slab 0
+  asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < NB; ++i) wf[0][i] = w_frag(0, 0, i);
+#pragma unroll
+  for (int i = 0; i < MB; ++i) xf[0][i] = x_frag(0, 0, i);
+
+  // MFMAs of register set P, meanwhile the fragments of the next step (set P ^ 1,
+  // step P ^ 1 of the slab at `base`) and, with COPY, the copies of slab `kt`.
+  auto step = [&](auto parity, auto with_copies, uint32_t base, int kt, uint32_t stage) {
+    constexpr int P = decltype(parity)::value;
+    constexpr bool COPY = decltype(with_copies)::value;
+#pragma unroll
+    for (int q = 0; q < kMfmas; ++q) {
+      __builtin_amdgcn_sched_barrier(0);
+      acc[q % NB][q / NB] = M::run(wf[P][q % NB], xf[P][q / NB], acc[q % NB][q / NB]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int z = 0; z < kReads; ++z)
+        if (z * kMfmas * 3 / 4 / kReads == q) {
+          if (z < NB) {
+            wf[P ^ 1][z] = w_frag(base, P ^ 1, z);
+          } else {
+            xf[P ^ 1][z - NB] = x_frag(base, P ^ 1, z - NB);
+          }
+        }
+      if constexpr (COPY) {
+#pragma unroll
+        for (int z = 0; z < CF::LOADS; ++z)
+          if (z * kMfmas * 3 / 4 / CF::LOADS == q) copy(z, kt, stage);
+      }
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  if (short_wave) {
-    wait_vmem<(S - 1) * kLoadsLo>();  // k-step 0
-  } else {
-    wait_vmem<(S - 1) * kLoadsHi>();
-  }
-  workgroup_barrier();
-#pragma unroll
-  for (int i = 0; i < MB; ++i) xf[i] = x_frag(0, i);
-#pragma unroll
-  for (int i = 0; i < NB; ++i) wf[i] = w_frag(0, i);
-  int stage = 0;  // stage of k-step kt
+  uint32_t stage = 0;  // of slab kt
   for (int kt = 0; kt < KT; ++kt) {
-    // The last iteration reads stage `next` too (harmless, unused): no branch.
-    const int next = stage + 1 == S ? 0 : stage + 1;
-    wait_next();
-    workgroup_barrier();
-    issue(stage, min(kt + S, KT - 1));
-    // The next W fragments go into a second register set first (every MFMA of
-    // this k-step reads the current ones); X fragment j is refilled from the
-    // next stage as soon as its last MFMA has issued.
-#pragma unroll
-    for (int i = 0; i < NB; ++i) wnext[i] = w_frag(next, i);
-#pragma unroll
-    for (int j = 0; j < MB; ++j) {
-#pragma unroll
-      for (int i = 0; i < NB; ++i) acc[i][j] = M::run(wf[i], xf[j], acc[i][j]);
-      xf[j] = x_frag(next, j);
-    }
-#pragma unroll
-    for (int i = 0; i < NB; ++i) wf[i] = wnext[i];
+    const uint32_t next = stage + 1 == S ? 0 : stage + 1;
+    step(std::integral_constant<int, 0>{}, std::false_type{}, stage * CF::SLAB, 0, 0);
+    wait_vmem<(S - 2) * CF::LOADS>();  // this wavefront's copies of slab kt + 1
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // (A last half slab has no second step.)
+    if (kt * kSlabK + kStepK < K)
+      step(std::integral_constant<int, 1>{}, std::true_type{}, next * CF::SLAB, kt + S, stage);
     stage = next;
   }
 
-  // ---- epilogue ----
-  // 1. Registers -> LDS: lane (c, g) holds Y[m][n .. n+3] of every 16 x 16
-  //    block; it adds the bias, rounds to T (as nn.Linear's output), applies
-  //    GELU if asked, and writes the four values into a row-major staging tile
-  //    (the LDS ring is free once every copy has landed and every wavefront
-  //    is past its last fragment read).
-  // 2. LDS -> HBM: the workgroup writes the 256 x BN tile in 16-byte chunks,
-  //    consecutive threads along a row, adding the residual for kEpiBiasAdd
-  //    with the same coalesced access.
-  const T* bias = reinterpret_cast<const T*>(a.bias);
-  Quad<T> bq[NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i)
-    bq[i] = *reinterpret_cast<const Quad<T>*>(bias + n_base + wn * CF::WN + 16 * i + 4 * g);
-  wait_vmem<0>();
-  workgroup_barrier();
-  T* tile = reinterpret_cast<T*>(smem);
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    const int col = wn * CF::WN + 16 * i + 4 * g;
-#pragma unroll
-    for (int j = 0; j < MB; ++j) {
-      const int row = wm * CF::WM + 16 * j + c;
-      Quad<T> out;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const T lin = static_cast<T>(acc[i][j][r] + static_cast<float>(bq[i][r]));
-        if constexpr (EPI == kEpiBiasGelu) {
-          out[r] = static_cast<T>(gelu_erf(static_cast<float>(lin)));
-        } else {
-          out[r] = lin;
-        }
-      }
-      *static_cast<Quad<T>*>(__builtin_assume_aligned(tile + row * CF::TILE_LD + col, 8)) = out;
-    }
-  }
-  workgroup_barrier();
-  constexpr int kRowChunks = BN / 8;  // 16-byte chunks per tile row
+  // ---- epilogue: bias, rounding to T (nn.Linear's output), GELU or residual;
+  // eight consecutive outputs of a row per lane and block pair ----
   typedef T Oct __attribute__((ext_vector_type(8)));
+  const T* bias = reinterpret_cast<const T*>(a.bias);
   const T* res = reinterpret_cast<const T*>(a.residual);
   T* Y = reinterpret_cast<T*>(a.y);
-  const int rows = min(CF::BM, a.M - m_base);
-  for (int q = tid; q < rows * kRowChunks; q += NT) {
-    const int row = q / kRowChunks;
-    const int ch = q - row * kRowChunks;
-    Oct v = *static_cast<const Oct*>(
-        __builtin_assume_aligned(tile + row * CF::TILE_LD + 8 * ch, 16));
-    const int64_t off = static_cast<int64_t>(m_base + row) * a.N + n_base + 8 * ch;
-    if constexpr (EPI == kEpiBiasAdd) {
-      const Oct rv = *reinterpret_cast<const Oct*>(res + off);
+  Quad<T> bq[NB];  // bias of the four outputs of block i
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        v[e] = static_cast<T>(static_cast<float>(v[e]) + static_cast<float>(rv[e]));
+  for (int i = 0; i < NB; ++i)
+    bq[i] = *reinterpret_cast<const Quad<T>*>(bias + n_base + wn * CF::WN + 16 * (i & ~1) + 8 * g +
+                                              4 * (i & 1));
+  // Row block by row block, so that the stores to the two halves of a 128-byte
+  // line follow each other, and past the L2 (non-temporal): Y is read next by another
+  // kernel, for which the L2 is written back and dropped in any case, and as
+  // dirty lines the stores push X and W out of it and wait to be written back at the
+  // end (16384 x 2304 x 768: 75 -> 58 us, FFN intermediate 16384 x 3072 x 768: 99 -> 83).
+#pragma unroll
+  for (int j = 0; j < MB; ++j) {
+    const int m = m_base + wm * CF::WM + 16 * j + c;
+    const int64_t row = static_cast<int64_t>(m) * a.N + n_base + wn * CF::WN + 8 * g;
+#pragma unroll
+    for (int i = 0; i < NB; i += 2) {
+      Oct out;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const T lin = static_cast<T>(acc[i + (e >> 2)][j][e & 3] +
+                                     static_cast<float>(bq[i + (e >> 2)][e & 3]));
+        if constexpr (EPI == kEpiBiasGelu) {
+          out[e] = static_cast<T>(gelu_erf(static_cast<float>(lin)));
+        } else {
+          out[e] = lin;
+        }
+      }
+      if (m >= a.M) continue;
+      if constexpr (EPI == kEpiBiasAdd) {
+        const Oct rv = *reinterpret_cast<const Oct*>(res + row + 16 * i);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          out[e] = static_cast<T>(static_cast<float>(out[e]) + static_cast<float>(rv[e]));
+      }
+      __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, out),
+                                  reinterpret_cast<u32x4_t*>(Y + row + 16 * i));
     }
-    *reinterpret_cast<Oct*>(Y + off) = v;
   }
+  wait_vmem<0>();  // no copy may land in LDS after the workgroup has ended
 }
 
 namespace {
 
-// Configurations: 256 x 192 tiles at one workgroup per CU (N % 192 == 0) and
-// 256 x 128 tiles at two (N % 128 == 0); for few rows, 64 x 128 tiles at three
-// workgroups per CU and 64 x 64 tiles at four, which give four times the tiles
-// of the 256-row forms (at 512 rows a 1536-wide projection has 96 and 192).
-using CfgWide = GemmConfig<192, 5, 1, 2, 2>;
-using CfgPair = GemmConfig<128, 3, 2, 2, 2>;
-using CfgEight = GemmConfig<192, 5, 1, 4, 2>;
-using CfgSmall = GemmConfig<128, 4, 3, 2, 2, 64>;
-using CfgTiny = GemmConfig<64, 4, 4, 2, 2, 64>;
-
-template <typename T, int EPI, typename CF>
-int launch_gemm(GemmArgs args, hipStream_t stream) {
-  constexpr auto* kernel = &gemm_kernel<T, EPI, CF>;
-  // The dynamic LDS limit is raised once per device (the attribute persists).
-  static std::atomic<uint64_t> raised{0};
-  int dev = 0;
-  hipError_t err = hipGetDevice(&dev);
-  if (err != hipSuccess) return static_cast<int>(err);
-  const uint64_t bit = dev < 64 ? (uint64_t{1} << dev) : 0;
-  if (bit == 0 || (raised.load(std::memory_order_acquire) & bit) == 0) {
-    err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, CF::LDS);
-    if (err == hipSuccess && bit != 0) raised.fetch_or(bit, std::memory_order_release);
-  }
-  if (err != hipSuccess) return static_cast<int>(err);
-  args.m_blocks = (args.M + CF::BM - 1) / CF::BM;
-  args.n_blocks = args.N / CF::BN;
-  // Each XCD walks a contiguous range of tiles.  Row-major ranges make every
-  // XCD read the whole of W (and its own rows of X), column-major ones the
-  // whole of X (and its own slice of W): take the order whose repeated operand
-  // is the smaller.
-  args.col_major = args.N > args.M ? 1 : 0;
-  const int64_t tiles = static_cast<int64_t>(args.m_blocks) * args.n_blocks;
-  const int64_t grid = ((tiles + 7) / 8) * 8;
-  if (grid > 0x7fffffff) return DFLASH_ERR_TOO_LARGE;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(CF::THREADS), CF::LDS,
-                     stream, args);
-  return static_cast<int>(hipGetLastError());
-}
+// Tile configurations (columns a multiple of the tile's; rows ragged).  Large tiles need the
+// fewest bytes per product and fill the chip from about 256 tiles; small ones, with
+// deeper rings, give few rows more workgroups.  gemm_cost says which is chosen.
+using Cfg128x192 = GemmConfig<128, 192, 2, 2, 2>;
+using Cfg128x128 = GemmConfig<128, 128, 2, 2, 2>;
+using Cfg256x192 = GemmConfig<256, 192, 4, 2, 1>;
+using Cfg64x128 = GemmConfig<64, 128, 2, 2, 2, 3>;
+using Cfg64x64 = GemmConfig<64, 64, 2, 2, 4>;
+using Cfg256x256 = GemmConfig<256, 256, 4, 2, 1>;
+using Cfg128x192Deep = GemmConfig<128, 192, 4, 2, 1, 4>;
+using Cfg128x128Deep = GemmConfig<128, 128, 4, 2, 1, 5>;
+using Cfg128x64 = GemmConfig<128, 64, 4, 1, 2, 3>;
+using Cfg64x64Deep = GemmConfig<64, 64, 2, 2, 2, 5>;
+using Cfg32x64 = GemmConfig<32, 64, 2, 2, 2, 6>;
 
 // CUs of the current device (cached per device; 256 if it cannot be read).
 int gemm_device_cus() {
@@ -443,42 +432,135 @@ int gemm_device_cus() {
   return cus;
 }
 
-// config: 0 = automatic, 1 = CfgWide, 2 = CfgPair, 3 = CfgEight, 4 = CfgSmall,
-// 5 = CfgTiny.  Automatic, for grids that fill at least half the CUs
-// (measured at M = 16384, fp16): CfgEight where N % 192 == 0 (QKV 71.7 us,
-// hidden-wide dense 24.5 us), except the GELU epilogue, whose VALU work
-// overlaps better at two workgroups per CU (CfgPair, FFN intermediate 108.5
-// against 117.6 us); CfgPair for N % 128 == 0 otherwise.
+template <typename T, int EPI, typename CF, bool FAR = false>
+int launch_gemm(GemmArgs args, hipStream_t stream) {
+  constexpr auto* kernel = &gemm_kernel<T, EPI, CF, FAR>;
+  // The dynamic LDS limit is raised once per device (the attribute persists).
+  static std::atomic<uint64_t> raised{0};
+  int dev = 0;
+  hipError_t err = hipGetDevice(&dev);
+  if (err != hipSuccess) return static_cast<int>(err);
+  const uint64_t bit = dev < 64 ? (uint64_t{1} << dev) : 0;
+  if (bit == 0 || (raised.load(std::memory_order_acquire) & bit) == 0) {
+    err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, CF::LDS);
+    if (err == hipSuccess && bit != 0) raised.fetch_or(bit, std::memory_order_release);
+  }
+  if (err != hipSuccess) return static_cast<int>(err);
+  args.m_blocks = (args.M + CF::BM - 1) / CF::BM;
+  args.n_blocks = args.N / CF::BN;
+  // XCDs along the rows and the columns: the split with the fewest rows of X and W
+  // for an XCD to read, among those whose largest range needs no more tiles than an
+  // even share rounded up to whole rounds of its CUs.
+  const int64_t tiles = static_cast<int64_t>(args.m_blocks) * args.n_blocks;
+  const int64_t round = (gemm_device_cus() + 7) / 8 * CF::WGS;
+  const int64_t rounds = ((tiles + 7) / 8 + round - 1) / round;
+  int64_t best = 0;
+  int64_t per_xcd = 0;
+  for (int gm = 1; gm <= 8; gm *= 2) {
+    const int gn = 8 / gm;
+    const int64_t mt = (args.m_blocks + gm - 1) / gm;
+    const int64_t nt = (args.n_blocks + gn - 1) / gn;
+    const int64_t read = mt * CF::BM + nt * CF::BN;
+    const bool even = (mt * nt + round - 1) / round <= rounds;
+    const int64_t score = read + (even ? 0 : (int64_t{1} << 40) + mt * nt);
+    if (best == 0 || score < best) {
+      best = score;
+      per_xcd = mt * nt;
+      args.xcds_m = gm;
+    }
+  }
+  const int64_t grid = 8 * per_xcd;
+  if (grid > 0x7fffffff) return DFLASH_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(CF::THREADS), CF::LDS,
+                     stream, args);
+  return static_cast<int>(hipGetLastError());
+}
+
+// Time of a launch in microseconds on a tile configuration, from its tiles and
+// its K:
+//   rounds of CUs * WGS tiles, each fixed + slabs * slab time; the slab time of a
+//   round with n tiles is slab1 + slab1_load * n / CUs while every CU has at most
+//   one tile, and reaches slab_full with WGS tiles on a CU; gelu: the GELU epilogue.
+// The constants are a least-squares fit (in the logarithm) to 900 timings (HIP
+// graphs of back-to-back calls over weights and activations that change from call to
+// call, fp16): K and N of 768- and 1536-wide layers (all four projections),
+// M = 16 .. 16384, every configuration.  Taking the configuration with the smallest
+// modelled time is then 0.6 % slower on average than taking the fastest one of
+// each shape, and at most 13 %.  The CUs are those of the device; the constants are
+// an MI355X's.
+struct GemmCost {
+  float fixed, slab1, slab1_load, slab_full, gelu;
+};
+
+template <typename CF>
+float gemm_cost(const GemmArgs& a, bool gelu, const GemmCost& c, int cus) {
+  const int64_t tiles = static_cast<int64_t>((a.M + CF::BM - 1) / CF::BM) * (a.N / CF::BN);
+  const int64_t cap = static_cast<int64_t>(cus) * CF::WGS;
+  const float slabs = static_cast<float>((a.K + kSlabK - 1) / kSlabK);
+  auto round = [&](int64_t n) {
+    const int64_t per_cu = (n + cus - 1) / cus;
+    float slab = c.slab1 + c.slab1_load * static_cast<float>(n < cus ? n : cus) / cus;
+    if constexpr (CF::WGS > 1)
+      slab += (c.slab_full - slab) * static_cast<float>(per_cu - 1) / (CF::WGS - 1);
+    return c.fixed + slabs * slab + (gelu ? c.gelu * per_cu / CF::WGS : 0.0f);
+  };
+  const int64_t full = tiles / cap;
+  const int64_t rest = tiles - full * cap;
+  return (full > 0 ? static_cast<float>(full) * round(cap) : 0.0f) + (rest > 0 ? round(rest) : 0.0f);
+}
+
+// config: 0 = automatic (the smallest modelled time), else the number of a
+// configuration.
 template <typename T, int EPI>
 int pick_config(const GemmArgs& args, int config, hipStream_t stream) {
-  const bool wide_ok = args.N % CfgWide::BN == 0;
-  const bool pair_ok = args.N % CfgPair::BN == 0;
-  if (config == 0 && !wide_ok && !pair_ok) {
-    config = 5;  // N % 64 == 0 only: the 64 x 64 tiles at every row count
-  } else if (config == 0) {
-    config = (wide_ok && !(EPI == kEpiBiasGelu && pair_ok)) ? 3 : 2;
-    // Few rows: when the 256-row grid would give fewer tiles than half the CUs,
-    // the 64-row forms (four times the tiles) are faster on the device, 64 x 64
-    // up to 1024 rows and 64 x 128 above (HIP-graph timings at 512 and 2048 rows:
-    // e.g. a 2304-wide projection of 512 x 768 in 7.0 against 17.6 us).
-    const int bn = config == 3 ? CfgEight::BN : CfgPair::BN;
-    const int64_t tiles = static_cast<int64_t>((args.M + 255) / 256) * (args.N / bn);
-    if (2 * tiles < gemm_device_cus()) config = (args.M <= 1024 || !pair_ok) ? 5 : 4;
+  // A tile's rows must lie within 32-bit byte offsets of its first one (256 rows
+  // of 2 K bytes); past that, 64 x 64 tiles with 64-bit copy addresses.
+  if (args.K >= (1 << 23) && config >= 0 && config <= 11)
+    return launch_gemm<T, EPI, Cfg64x64, true>(args, stream);
+  if (config == 0) {
+    const int cus = gemm_device_cus();
+    float best = 0.0f;
+    auto consider = [&](int number, auto cf, const GemmCost& cost) {
+      if (args.N % decltype(cf)::BN != 0) return;
+      const float us = gemm_cost<decltype(cf)>(args, EPI == kEpiBiasGelu, cost, cus);
+      if (config == 0 || us < best) {
+        config = number;
+        best = us;
+      }
+    };
+    consider(1, Cfg128x192{}, {3.72f, 0.684f, 0.175f, 1.339f, 3.54f});
+    consider(2, Cfg128x128{}, {3.15f, 0.580f, 0.193f, 0.879f, 2.41f});
+    consider(3, Cfg256x192{}, {5.39f, 0.832f, 0.390f, 0.0f, 2.99f});
+    consider(4, Cfg64x128{}, {3.27f, 0.298f, 0.028f, 0.571f, 1.07f});
+    consider(5, Cfg64x64{}, {3.89f, 0.386f, 0.0f, 0.619f, 0.98f});
+    consider(6, Cfg256x256{}, {6.84f, 0.994f, 0.505f, 0.0f, 3.69f});
+    consider(7, Cfg128x192Deep{}, {4.76f, 0.485f, 0.201f, 0.0f, 1.77f});
+    consider(8, Cfg128x128Deep{}, {4.10f, 0.382f, 0.110f, 0.0f, 1.11f});
+    consider(9, Cfg128x64{}, {3.22f, 0.282f, 0.052f, 0.563f, 0.88f});
+    consider(10, Cfg64x64Deep{}, {2.65f, 0.233f, 0.004f, 0.361f, 0.37f});
+    consider(11, Cfg32x64{}, {2.12f, 0.212f, 0.0f, 0.266f, 0.22f});
   }
+  auto fits = [&](auto cf) { return args.N % decltype(cf)::BN == 0; };
+#define DFLASH_GEMM_CASE(NUM, CF) \
+  case NUM:                       \
+    return fits(CF{}) ? launch_gemm<T, EPI, CF>(args, stream) : DFLASH_ERR_SHAPE;
   switch (config) {
-    case 1:
-      return wide_ok ? launch_gemm<T, EPI, CfgWide>(args, stream) : DFLASH_ERR_SHAPE;
-    case 2:
-      return pair_ok ? launch_gemm<T, EPI, CfgPair>(args, stream) : DFLASH_ERR_SHAPE;
-    case 3:
-      return wide_ok ? launch_gemm<T, EPI, CfgEight>(args, stream) : DFLASH_ERR_SHAPE;
-    case 4:
-      return pair_ok ? launch_gemm<T, EPI, CfgSmall>(args, stream) : DFLASH_ERR_SHAPE;
-    case 5:
-      return launch_gemm<T, EPI, CfgTiny>(args, stream);  // N % 64 == 0 is checked on entry
+    DFLASH_GEMM_CASE(1, Cfg128x192)
+    DFLASH_GEMM_CASE(2, Cfg128x128)
+    DFLASH_GEMM_CASE(3, Cfg256x192)
+    DFLASH_GEMM_CASE(4, Cfg64x128)
+    DFLASH_GEMM_CASE(5, Cfg64x64)
+    DFLASH_GEMM_CASE(6, Cfg256x256)
+    DFLASH_GEMM_CASE(7, Cfg128x192Deep)
+    DFLASH_GEMM_CASE(8, Cfg128x128Deep)
+    DFLASH_GEMM_CASE(9, Cfg128x64)
+    DFLASH_GEMM_CASE(10, Cfg64x64Deep)
+    DFLASH_GEMM_CASE(11, Cfg32x64)
     default:
       return DFLASH_ERR_SHAPE;
   }
+#undef DFLASH_GEMM_CASE
 }
 
 template <typename T>
@@ -508,7 +590,7 @@ extern "C" int dflash_linear_fwd(const void* x, const void* weight, const void* 
   if (M == 0) return DFLASH_OK;
   if (!x || !weight || !bias || !y) return DFLASH_ERR_NULL;
   if ((epilogue & 0xff) == DFLASH_GEMM_BIAS_ADD && !residual) return DFLASH_ERR_NULL;
-  if (N % 64 != 0 || K % kBK != 0) return DFLASH_ERR_SHAPE;
+  if (N % 64 != 0 || K % kStepK != 0) return DFLASH_ERR_SHAPE;
   if (static_cast<int64_t>(M) * K >= (int64_t{1} << 31) ||
       static_cast<int64_t>(M) * N >= (int64_t{1} << 31))
     return DFLASH_ERR_TOO_LARGE;
@@ -519,7 +601,7 @@ extern "C" int dflash_linear_fwd(const void* x, const void* weight, const void* 
   // Bits 8.. of `epilogue` select a tile configuration (0 = automatic).
   const int config = epilogue >> 8;
   epilogue &= 0xff;
-  GemmArgs args{x, weight, bias, residual, y, M, N, K, 0, 0};
+  GemmArgs args{x, weight, bias, residual, y, M, N, K, 0, 0, 1};
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == DFLASH_DTYPE_FP16) return dispatch_epilogue<_Float16>(args, epilogue, config, s);
   if (dtype == DFLASH_DTYPE_BF16) return dispatch_epilogue<__bf16>(args, epilogue, config, s);

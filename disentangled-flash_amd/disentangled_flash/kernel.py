@@ -392,8 +392,8 @@ class HipInferenceDisentangledSelfAttention(TorchInferenceDisentangledSelfAttent
         """Fused QKV projection ``[B, L, 3*H*d]`` (``_torch.py:284-297``).
 
         fp16/bf16 projections of a supported width run on the hand-written gfx950
-        GEMM (``dflash_linear_fwd``) where ``layers.hip_gemm_rows`` says so (by
-        row count and launch mode); others on ``F.linear``.
+        GEMM (``dflash_linear_fwd``) where ``layers.projection_on_hip`` says so; others
+        on ``F.linear``.
         """
 
         prep = self._prepared
@@ -402,7 +402,7 @@ class HipInferenceDisentangledSelfAttention(TorchInferenceDisentangledSelfAttent
                 "fused QKV projection is not prepared; call prepare_for_inference() first"
             )
         if layers.USE_HIP_GEMM and hidden_states.device.type == "cuda" \
-                and layers.hip_gemm_rows(hidden_states, prep.qkv_weight.shape[0]) \
+                and layers.projection_on_hip(hidden_states, prep.qkv_weight.shape[0]) \
                 and gemm_fits(prep.qkv_weight, prep.qkv_bias) \
                 and hidden_states.dtype == prep.qkv_weight.dtype:
             return linear_epilogue(gemm_rows(hidden_states), prep.qkv_weight, prep.qkv_bias, None,

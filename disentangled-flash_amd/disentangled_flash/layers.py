@@ -2,9 +2,9 @@
 
 ``DebertaV2SelfOutput`` and ``DebertaV2Output`` (reference ``_reference.py:101-112``
 and ``474-485``) both end in ``LayerNorm(dense(x) + input_tensor)``.  The HIP
-encoder keeps the dense projection on hipBLASLt (``F.linear`` with its bias
-epilogue) and replaces the separate residual add and LayerNorm with one
-kernel, ``disentangled_flash::add_layernorm``, which reads the projection and
+encoder runs the dense projection on the hand-written GEMM (:func:`linear_epilogue`)
+where :func:`projection_on_hip` says so, on ``F.linear`` otherwise, and replaces the
+separate residual add and LayerNorm with one kernel, ``disentangled_flash::add_layernorm``, which reads the projection and
 the residual once and writes the normalised row.
 
 The ``ConvLayer`` run after the first encoder layer (reference
@@ -86,26 +86,25 @@ def _layernorm_fake(x, weight, bias, eps):
 # an encoder is prepared and on every QKV projection.  A switch for A/B timing.
 USE_HIP_GEMM = True
 
-# Which GEMM runs an encoder projection, by rows (tokens, M = B*L), width and
-# launch mode.  Measured on whole encoders (12-layer base fp16, 24-layer xlarge
-# bf16) and per GEMM in HIP graphs:
-#   * HIP-graph replay: below HIP_GEMM_MIN_ROWS rows hipBLASLt (plus a separate
-#     GELU) is faster on the device, up to 1.5x at 512 rows; at 16384 rows the
-#     two tie;
-#   * eager, up to HIP_GEMM_EAGER_MAX_ROWS rows: the forward is bound by launch
-#     time, and an F.linear call costs about 19 us of hipBLASLt host time against
-#     a few for the hand-written GEMM.  For base-width projections (N or K at
-#     most HIP_GEMM_EAGER_MAX_WIDTH) that wins (1.85 -> 1.37 ms per forward at
-#     B*L <= 2048; 0.8-1.0 ms with the library's 64-row tiles at these rows);
-#     for the xlarge widths (N, K >= 1536) the hand-written kernel's device time
-#     outweighs it (3.47 -> 3.82 ms), and from about 4096 rows eager forwards are
-#     device-bound again.
-# So: the hand-written GEMM from HIP_GEMM_MIN_ROWS rows (QKV, attention-output
-# dense, FFN intermediate; the FFN output dense, K = 4 x hidden, stays on
-# hipBLASLt there), and in eager forwards up to HIP_GEMM_EAGER_MAX_ROWS rows at
-# base width; hipBLASLt otherwise, and always while a HIP graph is being captured
-# or torch.compile traces.  Checked on every call: the layer program binds the
-# fused steps once per bucket, while B varies per call.
+# Which GEMM runs an encoder projection (projection_on_hip).  Device times from HIP
+# graphs over changing operands, hand-written / hipBLASLt (+ its GELU pass), fp16, us:
+#   * width 768, 16384 rows: QKV 64.7 / 71.3, attention output 22.1 / 25.0, FFN
+#     intermediate + GELU 90 / 117, FFN output 77 / 71; 4096 rows: 18.1 / 19.7, 10.2 /
+#     11.9, 24.5 / 37.6, 25.3 / 27.1; 512 rows: 7.5 / 8.7, 5.4 / 7.6, 8.8 / 13.6, 11.8 /
+#     12.3.  So the hand-written GEMM runs everywhere but where K is long and the rows
+#     are few: the FFN output (K = 4 x hidden) below HIP_GEMM_LONG_K_ROWS rows, where its
+#     few tiles walk all of K one after the other (64 rows 11.7 / 7.4, and 20.1 / 14.8
+#     at width 1536);
+#   * there hip_gemm_rows decides: an eager forward is bound by launch time, and an
+#     F.linear call costs about 19 us of hipBLASLt host time against a few for the
+#     hand-written GEMM, so base-width projections (N or K at most
+#     HIP_GEMM_EAGER_MAX_WIDTH) of up to HIP_GEMM_EAGER_MAX_ROWS rows still take it
+#     eagerly, and hipBLASLt runs while a HIP graph is captured;
+#   * torch.compile traces hip_gemm_rows's rule for every projection: below
+#     HIP_GEMM_MIN_ROWS rows F.linear, which Inductor fuses.
+# Checked on every call: the layer program binds the fused steps once per bucket,
+# while B varies per call.
+HIP_GEMM_LONG_K_ROWS = 512
 HIP_GEMM_MIN_ROWS = 16384
 HIP_GEMM_EAGER_MAX_ROWS = 2048
 HIP_GEMM_EAGER_MAX_WIDTH = 768
@@ -116,8 +115,7 @@ _GRAPH_CHOICE = threading.local()
 @contextlib.contextmanager
 def graph_gemm_choice():
     """Eager forwards inside this block (on this thread) pick their GEMMs as HIP-graph
-    capture does (hipBLASLt below :data:`HIP_GEMM_MIN_ROWS` rows), so they reproduce a
-    captured bucket's replays bit for bit."""
+    capture does, so they reproduce a captured bucket's replays bit for bit."""
 
     saved = getattr(_GRAPH_CHOICE, "on", False)
     _GRAPH_CHOICE.on = True
@@ -142,8 +140,9 @@ def eager_small_gemm(x: torch.Tensor, n: int) -> bool:
 
 
 def hip_gemm_rows(x: torch.Tensor, n: int | None = None) -> bool:
-    """True if the projection of ``x`` (``[..., K]``) to ``n`` columns (default K)
-    runs on the hand-written GEMM."""
+    """The rule by rows and launch mode for the projection of ``x`` (``[..., K]``) to
+    ``n`` columns (default K): True from :data:`HIP_GEMM_MIN_ROWS` rows and in
+    launch-bound eager forwards (:func:`eager_small_gemm`)."""
 
     k = x.shape[-1]
     if k <= 0 or x.device.type != "cuda":
@@ -151,6 +150,19 @@ def hip_gemm_rows(x: torch.Tensor, n: int | None = None) -> bool:
     if x.numel() // k >= HIP_GEMM_MIN_ROWS:
         return True
     return eager_small_gemm(x, k if n is None else n)
+
+
+def projection_on_hip(x: torch.Tensor, n: int) -> bool:
+    """True if the projection of ``x`` (``[..., K]``) to ``n`` columns runs on the
+    hand-written GEMM (see the rules above)."""
+
+    k = x.shape[-1]
+    if k <= 0 or x.device.type != "cuda":
+        return False
+    if not torch.compiler.is_compiling() and (
+            k < 3 * n or x.numel() // k >= HIP_GEMM_LONG_K_ROWS):
+        return True
+    return hip_gemm_rows(x, n)
 
 
 # Tile configuration the encoder asks dflash_linear_fwd for (bits 8.. of its
@@ -256,26 +268,12 @@ def fusable_intermediate(module: nn.Module) -> bool:
 
 def intermediate_block(module: nn.Module, hidden_states: torch.Tensor) -> torch.Tensor:
     """``module(hidden_states)`` as one GEMM with the GELU in its epilogue, or the
-    module itself where :func:`hip_gemm_rows` says so."""
+    module itself where :func:`projection_on_hip` says so."""
 
-    if not hip_gemm_rows(hidden_states, module.dense.out_features):
+    if not projection_on_hip(hidden_states, module.dense.out_features):
         return module(hidden_states)
     return linear_epilogue(gemm_rows(hidden_states), module.dense.weight, module.dense.bias,
                            None, GEMM_BIAS_GELU)
-
-
-def output_block_gemm(module: nn.Module, hidden_states: torch.Tensor,
-                      input_tensor: torch.Tensor) -> torch.Tensor:
-    """``module(hidden_states, input_tensor)``: GEMM with the residual added in its
-    epilogue, then LayerNorm over the sum (one read of it instead of two); where
-    :func:`hip_gemm_rows` says so, hipBLASLt and the fused add + LayerNorm."""
-
-    if not hip_gemm_rows(hidden_states, module.dense.out_features):
-        return output_block(module, hidden_states, input_tensor)
-    summed = linear_epilogue(gemm_rows(hidden_states), module.dense.weight, module.dense.bias,
-                             gemm_rows(input_tensor), GEMM_BIAS_ADD)
-    norm = module.LayerNorm
-    return layernorm(summed, norm.weight, norm.bias, norm.eps)
 
 
 def fusable_output_block(module: nn.Module) -> bool:
@@ -305,24 +303,30 @@ def fusable_output_block(module: nn.Module) -> bool:
 
 def output_block(module: nn.Module, hidden_states: torch.Tensor,
                  input_tensor: torch.Tensor) -> torch.Tensor:
-    """``module(hidden_states, input_tensor)`` with the residual add and LayerNorm fused.
+    """``module(hidden_states, input_tensor)``: the dense projection, then one kernel for
+    the residual add and LayerNorm.
 
-    The dense runs on hipBLASLt, or in launch-bound eager forwards at base width
-    (:func:`eager_small_gemm`) on the hand-written GEMM with the residual in its
-    epilogue.  The caller checks :func:`fusable_output_block` once when the
-    encoder is prepared; this function is the hot path.
+    The residual is added there and not in the GEMM's epilogue: the same bytes, but
+    the epilogue's reads stand at the end of every tile (16384 x 768 x 768: GEMM 26.3 against
+    21.7 us, LayerNorm 10.8 against 13.1).  The caller checks
+    :func:`fusable_output_block` once when the encoder is prepared; this function is the
+    hot path.
     """
 
     dense = module.dense
     residual = input_tensor if input_tensor.is_contiguous() else input_tensor.contiguous()
     norm = module.LayerNorm
-    if USE_HIP_GEMM and eager_small_gemm(hidden_states, dense.out_features) \
-            and gemm_fits(dense.weight, dense.bias) and hidden_states.dtype == dense.weight.dtype:
-        summed = linear_epilogue(gemm_rows(hidden_states), dense.weight, dense.bias, residual,
-                                 GEMM_BIAS_ADD)
-        return layernorm(summed, norm.weight, norm.bias, norm.eps)
-    projected = F.linear(hidden_states, dense.weight, dense.bias)
+    if linear_fits(dense) and hidden_states.dtype == dense.weight.dtype \
+            and projection_on_hip(hidden_states, dense.out_features):
+        projected = linear_epilogue(gemm_rows(hidden_states), dense.weight, dense.bias, None,
+                                    GEMM_BIAS)
+    else:
+        projected = F.linear(hidden_states, dense.weight, dense.bias)
     return add_layernorm(projected, residual, norm.weight, norm.bias, norm.eps)
+
+
+# The attention output block runs the same form as the FFN's.
+output_block_gemm = output_block
 
 
 # ConvLayer.conv_act values the fused tail implements (DFLASH_ACT_* codes);

@@ -270,18 +270,18 @@ DFLASH_API int dflash_conv_layer_tail_fwd(const void* z, int z_dtype, const void
  *   y        : [M, N] row-major
  *   dtype    : fp16 or bf16 (fp32 is not supported: DFLASH_ERR_DTYPE)
  * N must be a multiple of 64 and K of 32 (DFLASH_ERR_SHAPE otherwise; every
- * projection of DeBERTa base/large/xlarge qualifies; the automatic configuration
- * runs the 64 x 64 tiles when N is a multiple of neither 128 nor 192, at any M);
+ * projection of DeBERTa base/large/xlarge qualifies);
  * x, weight, residual, y
  * 16-byte aligned, bias 8-byte aligned.  M == 0 is a no-op.
  *   epilogue : the code above in bits 0-7; bits 8 and up select a tile
- *              configuration (0 = automatic by N and epilogue): 1 = 256 x 192
- *              tiles, 4 wavefronts (N % 192 == 0); 2 = 256 x 128 at two workgroups per CU
- *              (N % 128 == 0); 3 = 256 x 192, 8 wavefronts (N % 192 == 0);
- *              4 = 64 x 128 at three per CU (N % 128 == 0); 5 = 64 x 64 at four
- *              per CU (N % 64 == 0).  The 64-row forms give four times the tiles
- *              for few rows.  A configuration that does not fit N returns
- *              DFLASH_ERR_SHAPE.
+ *              configuration (0 = automatic: the smallest modelled time for M, N, K
+ *              and epilogue), rows x columns of the tile: 1 = 128 x 192, two workgroups
+ *              per CU; 2 = 128 x 128, two per CU; 3 = 256 x 192; 4 = 64 x 128, two per
+ *              CU; 5 = 64 x 64, four per CU; 6 = 256 x 256; 7 = 128 x 192, 8
+ *              wavefronts, four slabs in LDS; 8 = 128 x 128, 8 wavefronts, five
+ *              slabs; 9 = 128 x 64, two per CU; 10 = 64 x 64, two per CU, five slabs;
+ *              11 = 32 x 64, two per CU, six slabs.  A configuration whose columns do
+ *              not divide N returns DFLASH_ERR_SHAPE.
  */
 DFLASH_API int dflash_linear_fwd(const void* x, const void* weight, const void* bias,
                                  const void* residual, void* y, int M, int N, int K,
