@@ -146,6 +146,16 @@ __device__ inline void copy16_to_lds_far(const void* src, uint32_t lds) {
       : "memory");
 }
 
+// 16-byte store at byte `off` of a buffer, written through the L2 (scope bit sc1).
+// For outputs that only a later kernel reads: as dirty lines they push out what this
+// kernel still reads and wait to be written back at its end.
+__device__ inline void store_through(__amdgpu_buffer_rsrc_t r, uint32_t off, u32x4_t v) {
+  constexpr int kSc1 = 16;
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, kSc1);
+}
+// Widest Y whose tile of up to 256 rows 32-bit byte offsets reach.
+constexpr int kMaxThroughN = 1 << 20;
+
 // Wait until at most N of this thread's vector-memory operations are pending.
 template <int N>
 __device__ inline void wait_vmem() {
@@ -192,6 +202,7 @@ struct GemmArgs {
   void* y;
   int M, N, K;
   int m_blocks, n_blocks;
+  int through;  // write Y through the L2 (store_through)
   int xcds_m;  // XCDs along the rows (1, 2, 4, 8); 8 / xcds_m along the columns
 };
 
@@ -362,11 +373,11 @@ __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) 
   for (int i = 0; i < NB; ++i)
     bq[i] = *reinterpret_cast<const Quad<T>*>(bias + n_base + wn * CF::WN + 16 * (i & ~1) + 8 * g +
                                               4 * (i & 1));
+  const int64_t y_base = static_cast<int64_t>(m_base) * a.N;
+  const auto yr = __builtin_amdgcn_make_buffer_rsrc(Y + y_base, static_cast<short>(0), 0x7fffffff,
+                                                    0x00020000);
   // Row block by row block, so that the stores to the two halves of a 128-byte
-  // line follow each other, and past the L2 (non-temporal): Y is read next by another
-  // kernel, for which the L2 is written back and dropped in any case, and as
-  // dirty lines the stores push X and W out of it and wait to be written back at the
-  // end (16384 x 2304 x 768: 75 -> 58 us, FFN intermediate 16384 x 3072 x 768: 99 -> 83).
+  // line follow each other.
 #pragma unroll
   for (int j = 0; j < MB; ++j) {
     const int m = m_base + wm * CF::WM + 16 * j + c;
@@ -391,8 +402,12 @@ __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) 
         for (int e = 0; e < 8; ++e)
           out[e] = static_cast<T>(static_cast<float>(out[e]) + static_cast<float>(rv[e]));
       }
-      __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, out),
-                                  reinterpret_cast<u32x4_t*>(Y + row + 16 * i));
+      if (a.through) {
+        store_through(yr, static_cast<uint32_t>(row + 16 * i - y_base) * 2u,
+                      __builtin_bit_cast(u32x4_t, out));
+      } else {
+        *reinterpret_cast<Oct*>(Y + row + 16 * i) = out;
+      }
     }
   }
   wait_vmem<0>();  // no copy may land in LDS after the workgroup has ended
@@ -449,6 +464,11 @@ int launch_gemm(GemmArgs args, hipStream_t stream) {
   if (err != hipSuccess) return static_cast<int>(err);
   args.m_blocks = (args.M + CF::BM - 1) / CF::BM;
   args.n_blocks = args.N / CF::BN;
+  // Y through the L2 unless it is large: 12 layers of 4096 rows, 768 wide (Y of 6 to 25 MB)
+  // 1416 us, left in the L2 1462, non-temporal 1508; one layer of 16384 rows, with QKV
+  // and FFN outputs of 75 and 100 MB, 357, 349 and 363 us.
+  args.through = args.N <= kMaxThroughN &&
+                 static_cast<int64_t>(args.M) * args.N * 2 < (int64_t{48} << 20);
   // XCDs along the rows and the columns: the split with the fewest rows of X and W
   // for an XCD to read, among those whose largest range needs no more tiles than an
   // even share rounded up to whole rounds of its CUs.
@@ -601,7 +621,7 @@ extern "C" int dflash_linear_fwd(const void* x, const void* weight, const void* 
   // Bits 8.. of `epilogue` select a tile configuration (0 = automatic).
   const int config = epilogue >> 8;
   epilogue &= 0xff;
-  GemmArgs args{x, weight, bias, residual, y, M, N, K, 0, 0, 1};
+  GemmArgs args{x, weight, bias, residual, y, M, N, K, 0, 0, 0, 1};
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == DFLASH_DTYPE_FP16) return dispatch_epilogue<_Float16>(args, epilogue, config, s);
   if (dtype == DFLASH_DTYPE_BF16) return dispatch_epilogue<__bf16>(args, epilogue, config, s);
