@@ -68,6 +68,7 @@
 
 #include "device_common.h"
 #include "dflash.h"
+#include "layernorm.h"
 
 namespace dflash {
 
@@ -79,6 +80,7 @@ constexpr int kSlabK = 2 * kStepK;    // k of one slab (128-byte rows)
 constexpr int kEpiBias = 0;
 constexpr int kEpiBiasGelu = 1;
 constexpr int kEpiBiasAdd = 2;
+constexpr int kEpiPartial = 3;  // fp32 sums of one of `splits` ranges of K, no bias
 
 // Chunk permutation of slab row r: 16-byte chunk k of the row sits at position
 // k ^ slab_swizzle(r).  Eight consecutive rows hit eight different chunks of a
@@ -203,6 +205,7 @@ struct GemmArgs {
   int M, N, K;
   int m_blocks, n_blocks;
   int through;  // write Y through the L2 (store_through)
+  int splits;   // ranges of K (kEpiPartial; y is fp32 [splits, M, N]), else 1
   int xcds_m;  // XCDs along the rows (1, 2, 4, 8); 8 / xcds_m along the columns
 };
 
@@ -229,25 +232,31 @@ __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) 
   // Tile of this workgroup (see the file comment): the tile ranges of XCD p % 8,
   // columns fastest.
   const int p = blockIdx.x;
+  const int split = EPI == kEpiPartial ? (p >> 3) % a.splits : 0;
+  const int index = EPI == kEpiPartial ? (p >> 3) / a.splits : p >> 3;
   const int xm = (p & 7) % a.xcds_m;
   const int xn = (p & 7) / a.xcds_m;
   const int m_lo = a.m_blocks * xm / a.xcds_m;
   const int n_lo = a.n_blocks * xn * a.xcds_m / 8;
   const int cols = a.n_blocks * (xn + 1) * a.xcds_m / 8 - n_lo;
-  const int mt = (p >> 3) / max(cols, 1);
+  const int mt = index / max(cols, 1);
   const int mb = m_lo + mt;
-  const int nb = n_lo + (p >> 3) - mt * cols;
+  const int nb = n_lo + index - mt * cols;
   if (cols == 0 || mb >= a.m_blocks * (xm + 1) / a.xcds_m) return;  // ranges differ in size
   const int m_base = mb * CF::BM;
   const int n_base = nb * CF::BN;
-  const int K = a.K;
-  const int KT = (K + kSlabK - 1) / kSlabK;  // slabs (the last may be half: K is a multiple of 32)
-  const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
+  const int ld = a.K;  // row stride of X and W
+  const int all_slabs = (a.K + kSlabK - 1) / kSlabK;  // (the last may be half: K % 32 == 0)
+  const int slab_lo = EPI == kEpiPartial ? all_slabs * split / a.splits : 0;
+  const int KT = EPI == kEpiPartial ? all_slabs * (split + 1) / a.splits - slab_lo : all_slabs;
+  const int K = min(a.K - slab_lo * kSlabK, KT * kSlabK);  // of this workgroup
+  const uint32_t row_bytes = static_cast<uint32_t>(ld) * 2u;
   const int rows = min(CF::BM, a.M - m_base);
-  const T* X = reinterpret_cast<const T*>(a.x) + static_cast<int64_t>(m_base) * K;
-  const T* W = reinterpret_cast<const T*>(a.w) + static_cast<int64_t>(n_base) * K;
-  const uint32_t x_bytes = static_cast<uint32_t>(rows) * row_bytes;
-  const uint32_t w_bytes = static_cast<uint32_t>(CF::BN) * row_bytes;
+  const T* X = reinterpret_cast<const T*>(a.x) + static_cast<int64_t>(m_base) * ld + slab_lo * kSlabK;
+  const T* W = reinterpret_cast<const T*>(a.w) + static_cast<int64_t>(n_base) * ld + slab_lo * kSlabK;
+  const uint32_t skipped = static_cast<uint32_t>(slab_lo) * (kSlabK * 2);
+  const uint32_t x_bytes = static_cast<uint32_t>(rows) * row_bytes - skipped;
+  const uint32_t w_bytes = static_cast<uint32_t>(CF::BN) * row_bytes - skipped;
 
   // Copy j of a slab fetches eight slab rows (8 lanes a row): row and source
   // chunk of this lane, and its byte offset from the tile's first row.
@@ -278,7 +287,7 @@ __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) 
       // last 32 (their products are not computed).
       const int r = is_x ? min(slab_row(jj), rows - 1) : w_row(slab_row(jj));
       const int k = min(slab_at(min(kt, KT - 1)) * kSlabK + chunk_of(slab_row(jj)) * 8, K - 8);
-      copy16_to_lds_far((is_x ? X : W) + static_cast<int64_t>(r) * K + k, dst);
+      copy16_to_lds_far((is_x ? X : W) + static_cast<int64_t>(r) * ld + k, dst);
     } else {
       const uint32_t bytes = kt < KT ? (is_x ? x_bytes : w_bytes) : 0u;
       const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -362,6 +371,20 @@ __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) 
     stage = next;
   }
 
+  if constexpr (EPI == kEpiPartial) {
+    float* part = reinterpret_cast<float*>(a.y) + static_cast<int64_t>(split) * a.M * a.N;
+#pragma unroll
+    for (int j = 0; j < MB; ++j) {
+      const int m = m_base + wm * CF::WM + 16 * j + c;
+      if (m >= a.M) continue;
+      float* row = part + static_cast<int64_t>(m) * a.N + n_base + wn * CF::WN + 8 * g;
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+        *reinterpret_cast<f32x4_t*>(row + 16 * (i & ~1) + 4 * (i & 1)) = acc[i][j];
+    }
+    wait_vmem<0>();
+    return;
+  }
   // ---- epilogue: bias, rounding to T (nn.Linear's output), GELU or residual;
   // eight consecutive outputs of a row per lane and block pair ----
   typedef T Oct __attribute__((ext_vector_type(8)));
@@ -490,7 +513,7 @@ int launch_gemm(GemmArgs args, hipStream_t stream) {
       args.xcds_m = gm;
     }
   }
-  const int64_t grid = 8 * per_xcd;
+  const int64_t grid = 8 * per_xcd * args.splits;
   if (grid > 0x7fffffff) return DFLASH_ERR_TOO_LARGE;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(CF::THREADS), CF::LDS,
                      stream, args);
@@ -515,9 +538,11 @@ struct GemmCost {
 
 template <typename CF>
 float gemm_cost(const GemmArgs& a, bool gelu, const GemmCost& c, int cus) {
-  const int64_t tiles = static_cast<int64_t>((a.M + CF::BM - 1) / CF::BM) * (a.N / CF::BN);
+  const int64_t tiles =
+      static_cast<int64_t>((a.M + CF::BM - 1) / CF::BM) * (a.N / CF::BN) * a.splits;
   const int64_t cap = static_cast<int64_t>(cus) * CF::WGS;
-  const float slabs = static_cast<float>((a.K + kSlabK - 1) / kSlabK);
+  const int all_slabs = (a.K + kSlabK - 1) / kSlabK;
+  const float slabs = static_cast<float>((all_slabs + a.splits - 1) / a.splits);
   auto round = [&](int64_t n) {
     const int64_t per_cu = (n + cus - 1) / cus;
     float slab = c.slab1 + c.slab1_load * static_cast<float>(n < cus ? n : cus) / cus;
@@ -530,25 +555,20 @@ float gemm_cost(const GemmArgs& a, bool gelu, const GemmCost& c, int cus) {
   return (full > 0 ? static_cast<float>(full) * round(cap) : 0.0f) + (rest > 0 ? round(rest) : 0.0f);
 }
 
-// config: 0 = automatic (the smallest modelled time), else the number of a
-// configuration.
-template <typename T, int EPI>
-int pick_config(const GemmArgs& args, int config, hipStream_t stream) {
-  // A tile's rows must lie within 32-bit byte offsets of its first one (256 rows
-  // of 2 K bytes); past that, 64 x 64 tiles with 64-bit copy addresses.
-  if (args.K >= (1 << 23) && config >= 0 && config <= 11)
-    return launch_gemm<T, EPI, Cfg64x64, true>(args, stream);
-  if (config == 0) {
-    const int cus = gemm_device_cus();
-    float best = 0.0f;
-    auto consider = [&](int number, auto cf, const GemmCost& cost) {
-      if (args.N % decltype(cf)::BN != 0) return;
-      const float us = gemm_cost<decltype(cf)>(args, EPI == kEpiBiasGelu, cost, cus);
-      if (config == 0 || us < best) {
-        config = number;
-        best = us;
-      }
-    };
+// The configuration with the smallest modelled time; with splits > 1 among the ones
+// built for partial sums.
+int best_config(const GemmArgs& args, bool gelu, float* us) {
+  const int cus = gemm_device_cus();
+  int config = 0;
+  auto consider = [&](int number, auto cf, const GemmCost& cost) {
+    if (args.N % decltype(cf)::BN != 0) return;
+    const float t = gemm_cost<decltype(cf)>(args, gelu, cost, cus);
+    if (config == 0 || t < *us) {
+      config = number;
+      *us = t;
+    }
+  };
+  if (args.splits == 1) {
     consider(1, Cfg128x192{}, {3.72f, 0.684f, 0.175f, 1.339f, 3.54f});
     consider(2, Cfg128x128{}, {3.15f, 0.580f, 0.193f, 0.879f, 2.41f});
     consider(3, Cfg256x192{}, {5.39f, 0.832f, 0.390f, 0.0f, 2.99f});
@@ -557,9 +577,23 @@ int pick_config(const GemmArgs& args, int config, hipStream_t stream) {
     consider(6, Cfg256x256{}, {6.84f, 0.994f, 0.505f, 0.0f, 3.69f});
     consider(7, Cfg128x192Deep{}, {4.76f, 0.485f, 0.201f, 0.0f, 1.77f});
     consider(8, Cfg128x128Deep{}, {4.10f, 0.382f, 0.110f, 0.0f, 1.11f});
-    consider(9, Cfg128x64{}, {3.22f, 0.282f, 0.052f, 0.563f, 0.88f});
-    consider(10, Cfg64x64Deep{}, {2.65f, 0.233f, 0.004f, 0.361f, 0.37f});
-    consider(11, Cfg32x64{}, {2.12f, 0.212f, 0.0f, 0.266f, 0.22f});
+  }
+  consider(9, Cfg128x64{}, {3.22f, 0.282f, 0.052f, 0.563f, 0.88f});
+  consider(10, Cfg64x64Deep{}, {2.65f, 0.233f, 0.004f, 0.361f, 0.37f});
+  consider(11, Cfg32x64{}, {2.12f, 0.212f, 0.0f, 0.266f, 0.22f});
+  return config;
+}
+
+// config: 0 = automatic, else the number of a configuration.
+template <typename T, int EPI>
+int pick_config(const GemmArgs& args, int config, hipStream_t stream) {
+  // A tile's rows must lie within 32-bit byte offsets of its first one (256 rows
+  // of 2 K bytes); past that, 64 x 64 tiles with 64-bit copy addresses.
+  if (args.K >= (1 << 23) && config >= 0 && config <= 11)
+    return launch_gemm<T, EPI, Cfg64x64, true>(args, stream);
+  if (config == 0) {
+    float us = 0.0f;
+    config = best_config(args, EPI == kEpiBiasGelu, &us);
   }
   auto fits = [&](auto cf) { return args.N % decltype(cf)::BN == 0; };
 #define DFLASH_GEMM_CASE(NUM, CF) \
@@ -597,6 +631,55 @@ int dispatch_epilogue(const GemmArgs& args, int epilogue, int config, hipStream_
   }
 }
 
+template <typename T>
+int launch_partial(const GemmArgs& args, int config, hipStream_t stream) {
+  switch (config) {
+    case 9:
+      return launch_gemm<T, kEpiPartial, Cfg128x64>(args, stream);
+    case 10:
+      return launch_gemm<T, kEpiPartial, Cfg64x64Deep>(args, stream);
+    case 11:
+      return launch_gemm<T, kEpiPartial, Cfg32x64>(args, stream);
+    default:
+      return DFLASH_ERR_SHAPE;
+  }
+}
+
+constexpr int kMaxSplits = 8;
+
+// Ranges of K (1, 2, 4 or 8) of an output block's projection, and the
+// configuration for more than one.  With few rows the tiles leave most CUs idle and
+// walk all of K one after the other; the LayerNorm reads every row anyway and adds
+// the ranges' sums on the way.  Split where the modelled time, with the partial sums
+// written and read at 4 MB a microsecond, is at least a microsecond less.  Projection and
+// LayerNorm together, unsplit / split, us: 64 x 768 x 3072 15.5 / 8.9 (8 ranges),
+// 512 x 768 x 3072 15.8 / 13.6 (2), 64 x 1536 x 6144 24.6 / 14.6 (8), 64 x 768 x 768 8.5 / 7.2
+// (2); from 1024 rows none is split.
+int output_splits(int M, int N, int K, int* config) {
+  *config = 0;
+  GemmArgs args{};
+  args.M = M;
+  args.N = N;
+  args.K = K;
+  args.splits = 1;
+  float best = 0.0f;
+  if (K >= (1 << 23) || best_config(args, false, &best) == 0) return 1;
+  best -= 1.0f;
+  int splits = 1;
+  for (int s = 2; s <= kMaxSplits && K / s >= 4 * kSlabK; s *= 2) {
+    args.splits = s;
+    float us = 0.0f;
+    const int number = best_config(args, false, &us);
+    us += 8.0f * s * static_cast<float>(M) * static_cast<float>(N) / 4e6f;
+    if (number != 0 && us < best) {
+      best = us;
+      splits = s;
+      *config = number;
+    }
+  }
+  return splits;
+}
+
 }  // namespace
 
 }  // namespace dflash
@@ -621,9 +704,52 @@ extern "C" int dflash_linear_fwd(const void* x, const void* weight, const void* 
   // Bits 8.. of `epilogue` select a tile configuration (0 = automatic).
   const int config = epilogue >> 8;
   epilogue &= 0xff;
-  GemmArgs args{x, weight, bias, residual, y, M, N, K, 0, 0, 0, 1};
+  GemmArgs args{x, weight, bias, residual, y, M, N, K, 0, 0, 0, 1, 1};
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == DFLASH_DTYPE_FP16) return dispatch_epilogue<_Float16>(args, epilogue, config, s);
   if (dtype == DFLASH_DTYPE_BF16) return dispatch_epilogue<__bf16>(args, epilogue, config, s);
   return DFLASH_ERR_DTYPE;
+}
+
+extern "C" size_t dflash_output_block_workspace_bytes(int M, int N, int K) {
+  if (M < 1 || N < 1 || K < 1) return 0;
+  int config = 0;
+  const int splits = output_splits(M, N, K, &config);
+  return static_cast<size_t>(M) * N * (splits > 1 ? sizeof(float) * splits : 2);
+}
+
+extern "C" int dflash_output_block_fwd(const void* x, const void* weight, const void* bias,
+                                       const void* residual, const void* gamma, const void* beta,
+                                       void* out, int M, int N, int K, float eps, int dtype,
+                                       void* workspace, size_t workspace_bytes, void* stream) {
+  if (M < 0 || N < 1 || K < 1) return DFLASH_ERR_SHAPE;
+  if (M == 0) return DFLASH_OK;
+  if (!residual || !workspace) return DFLASH_ERR_NULL;
+  if (workspace_bytes < dflash_output_block_workspace_bytes(M, N, K)) return DFLASH_ERR_WORKSPACE;
+  if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return DFLASH_ERR_ALIGN;
+  int config = 0;
+  const int splits = output_splits(M, N, K, &config);
+  if (splits == 1) {
+    const int rc = dflash_linear_fwd(x, weight, bias, nullptr, workspace, M, N, K,
+                                     DFLASH_GEMM_BIAS, dtype, stream);
+    if (rc != DFLASH_OK) return rc;
+    return dflash_add_layernorm_fwd(workspace, residual, gamma, beta, out, M, N, eps, dtype,
+                                    stream);
+  }
+  if (!x || !weight || !bias || !gamma || !beta || !out) return DFLASH_ERR_NULL;
+  if (N % 64 != 0 || K % kStepK != 0 || N > 4096) return DFLASH_ERR_SHAPE;
+  if (dtype != DFLASH_DTYPE_FP16 && dtype != DFLASH_DTYPE_BF16) return DFLASH_ERR_DTYPE;
+  if (static_cast<int64_t>(M) * K >= (int64_t{1} << 31)) return DFLASH_ERR_TOO_LARGE;
+  const uintptr_t wide = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(weight);
+  const uintptr_t quad = reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(residual) |
+                         reinterpret_cast<uintptr_t>(gamma) | reinterpret_cast<uintptr_t>(beta) |
+                         reinterpret_cast<uintptr_t>(out);
+  if (wide % 16 != 0 || quad % 8 != 0) return DFLASH_ERR_ALIGN;
+  GemmArgs args{x, weight, nullptr, nullptr, workspace, M, N, K, 0, 0, 0, splits, 1};
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rc = dtype == DFLASH_DTYPE_FP16 ? launch_partial<_Float16>(args, config, s)
+                                            : launch_partial<__bf16>(args, config, s);
+  if (rc != DFLASH_OK) return rc;
+  return launch_partials_layernorm(static_cast<const float*>(workspace), splits, bias, residual,
+                                   gamma, beta, out, M, N, eps, dtype, s);
 }

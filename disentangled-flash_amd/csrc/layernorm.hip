@@ -18,6 +18,7 @@
 #include <stdint.h>
 
 #include "dflash.h"
+#include "layernorm.h"
 
 namespace dflash {
 namespace {
@@ -257,7 +258,130 @@ int dispatch_ln(const void* x, const void* r, const void* gamma, const void* bet
   }
 }
 
+// Residual add + LayerNorm of a projection whose K range was split: one
+// wavefront per row adds the SPLITS fp32 partial sums in order, then the bias, and
+// rounds to T as nn.Linear's output is; the rest is add_layernorm_kernel.  Few rows (that is
+// when a projection is split), so it is bound by latency: every load of the row is in
+// flight before the first sum.  VPL = 4-element chunks per lane.
+template <typename T, int VPL, int SPLITS>
+__global__ __launch_bounds__(64) void partials_layernorm_kernel(
+    const float* __restrict__ part, const T* __restrict__ bias, const T* __restrict__ r,
+    const T* __restrict__ gamma, const T* __restrict__ beta, T* __restrict__ y, int rows,
+    int hidden, float eps) {
+  using V = typename Vec4<T>::type;
+  typedef float F4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x;
+  const int row = blockIdx.x;
+  const int64_t base = static_cast<int64_t>(row) * hidden;
+  const int64_t step = static_cast<int64_t>(rows) * hidden;
+  const int nvec = hidden >> 2;
+
+  F4 p[VPL][SPLITS];
+  V bb[VPL], rr[VPL], gg[VPL], tt[VPL];
+#pragma unroll
+  for (int k = 0; k < VPL; ++k) {
+    const int v = lane + 64 * k;
+    if (v < nvec) {
+#pragma unroll
+      for (int s = 0; s < SPLITS; ++s)
+        p[k][s] = *reinterpret_cast<const F4*>(part + s * step + base + 4 * v);
+      bb[k] = *reinterpret_cast<const V*>(bias + 4 * v);
+      rr[k] = *reinterpret_cast<const V*>(r + base + 4 * v);
+      gg[k] = *reinterpret_cast<const V*>(gamma + 4 * v);
+      tt[k] = *reinterpret_cast<const V*>(beta + 4 * v);
+    }
+  }
+  float s[VPL][4];
+  float sum = 0.0f;
+#pragma unroll
+  for (int k = 0; k < VPL; ++k) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[k][e] = 0.0f;
+    if (lane + 64 * k < nvec) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float x = p[k][0][e];
+#pragma unroll
+        for (int sp = 1; sp < SPLITS; ++sp) x += p[k][sp][e];
+        const T lin = static_cast<T>(x + static_cast<float>(bb[k][e]));
+        s[k][e] = static_cast<float>(
+            static_cast<T>(static_cast<float>(lin) + static_cast<float>(rr[k][e])));
+        sum += s[k][e];
+      }
+    }
+  }
+  const float inv_h = 1.0f / static_cast<float>(hidden);
+  const float mean = wave_sum(sum) * inv_h;
+  float sq = 0.0f;
+#pragma unroll
+  for (int k = 0; k < VPL; ++k) {
+    if (lane + 64 * k < nvec) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float d = s[k][e] - mean;
+        sq += d * d;
+      }
+    }
+  }
+  const float rstd = rsqrtf(wave_sum(sq) * inv_h + eps);
+#pragma unroll
+  for (int k = 0; k < VPL; ++k) {
+    const int v = lane + 64 * k;
+    if (v < nvec) {
+      V out;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        out[e] = static_cast<T>((s[k][e] - mean) * rstd * static_cast<float>(gg[k][e]) +
+                                static_cast<float>(tt[k][e]));
+      *reinterpret_cast<V*>(y + base + 4 * v) = out;
+    }
+  }
+}
+
+template <typename T, int VPL>
+int launch_partials(const float* part, int splits, const void* bias, const void* residual,
+                    const void* gamma, const void* beta, void* out, int rows, int hidden,
+                    float eps, hipStream_t stream) {
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(64), 0, stream, part, static_cast<const T*>(bias),
+                       static_cast<const T*>(residual), static_cast<const T*>(gamma),
+                       static_cast<const T*>(beta), static_cast<T*>(out), rows, hidden, eps);
+    return static_cast<int>(hipGetLastError());
+  };
+  switch (splits) {
+    case 2: return go(&partials_layernorm_kernel<T, VPL, 2>);
+    case 4: return go(&partials_layernorm_kernel<T, VPL, 4>);
+    case 8: return go(&partials_layernorm_kernel<T, VPL, 8>);
+    default: return DFLASH_ERR_SHAPE;
+  }
+}
+
+template <typename T>
+int dispatch_partials(const float* part, int splits, const void* bias, const void* residual,
+                      const void* gamma, const void* beta, void* out, int rows, int hidden,
+                      float eps, hipStream_t stream) {
+#define DFLASH_PARTIALS(V) \
+  launch_partials<T, V>(part, splits, bias, residual, gamma, beta, out, rows, hidden, eps, stream)
+  if (hidden <= 768) return DFLASH_PARTIALS(3);
+  if (hidden <= 1024) return DFLASH_PARTIALS(4);
+  if (hidden <= 1536) return DFLASH_PARTIALS(6);
+  return DFLASH_PARTIALS(16);
+#undef DFLASH_PARTIALS
+}
+
 }  // namespace
+
+int launch_partials_layernorm(const float* part, int splits, const void* bias,
+                              const void* residual, const void* gamma, const void* beta,
+                              void* out, int rows, int hidden, float eps, int dtype,
+                              hipStream_t stream) {
+  return dtype == DFLASH_DTYPE_FP16
+             ? dispatch_partials<_Float16>(part, splits, bias, residual, gamma, beta, out, rows,
+                                           hidden, eps, stream)
+             : dispatch_partials<__bf16>(part, splits, bias, residual, gamma, beta, out, rows,
+                                         hidden, eps, stream);
+}
+
 }  // namespace dflash
 
 using namespace dflash;

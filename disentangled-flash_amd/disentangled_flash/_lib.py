@@ -100,6 +100,15 @@ def _bind(lib: ctypes.CDLL) -> None:
         _c_int, _c_int, _c_int, _c_int, _c_int,                  # M, N, K, epilogue, dtype
         _c_void_p,                                               # stream
     ]
+    lib.dflash_output_block_workspace_bytes.restype = ctypes.c_size_t
+    lib.dflash_output_block_workspace_bytes.argtypes = [_c_int, _c_int, _c_int]  # M, N, K
+    lib.dflash_output_block_fwd.restype = _c_int
+    lib.dflash_output_block_fwd.argtypes = [
+        _c_void_p, _c_void_p, _c_void_p, _c_void_p,              # x, weight, bias, residual
+        _c_void_p, _c_void_p, _c_void_p,                         # gamma, beta, out
+        _c_int, _c_int, _c_int, _c_float, _c_int,                # M, N, K, eps, dtype
+        _c_void_p, ctypes.c_size_t, _c_void_p,                   # workspace, bytes, stream
+    ]
     lib.dflash_error_string.restype = ctypes.c_char_p
     lib.dflash_error_string.argtypes = [_c_int]
     lib.dflash_abi_version.restype = _c_int

@@ -1,9 +1,8 @@
 """HIP-graph buckets: replay a prepared encoder forward without host launch cost.
 
 At small batches the eager encoder is bound by the host, not the GPU: each
-layer issues four hipBLASLt GEMMs (about 20 us of host time each on ROCm), the
-attention and LayerNorm ops and a few torch elementwise kernels, so a 12-layer
-forward costs about 1.9 ms of host time whatever the batch.  A HIP graph
+layer issues its projections, the attention and the LayerNorms from Python, so a
+12-layer forward costs about a millisecond of host time whatever the batch.  A HIP graph
 records the whole launch sequence of one (batch, bucket length) once and
 replays it with a single host call.
 
@@ -59,7 +58,7 @@ class DebertaGraphBucket:
         side.wait_stream(torch.cuda.current_stream(weight.device))
         with torch.inference_mode(), torch.cuda.stream(side):
             # Library handles and workspaces exist before capture: the warm-up runs the
-            # kernels the capture will record (capture picks hipBLASLt for few rows).
+            # kernels the capture will record.
             with layers.graph_gemm_choice():
                 for _ in range(max(1, warmup)):
                     run()

@@ -86,25 +86,17 @@ def _layernorm_fake(x, weight, bias, eps):
 # an encoder is prepared and on every QKV projection.  A switch for A/B timing.
 USE_HIP_GEMM = True
 
-# Which GEMM runs an encoder projection (projection_on_hip).  Device times from HIP
-# graphs over changing operands, hand-written / hipBLASLt (+ its GELU pass), fp16, us:
+# Which GEMM runs an encoder projection (projection_on_hip): the hand-written one where
+# it fits (gemm_fits).  Device times from HIP graphs over changing operands, hand-written /
+# hipBLASLt (+ its GELU pass, + the fused add + LayerNorm for the output blocks), fp16, us:
 #   * width 768, 16384 rows: QKV 64.7 / 71.3, attention output 22.1 / 25.0, FFN
-#     intermediate + GELU 90 / 117, FFN output 77 / 71; 4096 rows: 18.1 / 19.7, 10.2 /
-#     11.9, 24.5 / 37.6, 25.3 / 27.1; 512 rows: 7.5 / 8.7, 5.4 / 7.6, 8.8 / 13.6, 11.8 /
-#     12.3.  So the hand-written GEMM runs everywhere but where K is long and the rows
-#     are few: the FFN output (K = 4 x hidden) below HIP_GEMM_LONG_K_ROWS rows, where its
-#     few tiles walk all of K one after the other (64 rows 11.7 / 7.4, and 20.1 / 14.8
-#     at width 1536);
-#   * there hip_gemm_rows decides: an eager forward is bound by launch time, and an
-#     F.linear call costs about 19 us of hipBLASLt host time against a few for the
-#     hand-written GEMM, so base-width projections (N or K at most
-#     HIP_GEMM_EAGER_MAX_WIDTH) of up to HIP_GEMM_EAGER_MAX_ROWS rows still take it
-#     eagerly, and hipBLASLt runs while a HIP graph is captured;
-#   * torch.compile traces hip_gemm_rows's rule for every projection: below
-#     HIP_GEMM_MIN_ROWS rows F.linear, which Inductor fuses.
-# Checked on every call: the layer program binds the fused steps once per bucket,
-# while B varies per call.
-HIP_GEMM_LONG_K_ROWS = 512
+#     intermediate + GELU 90 / 117, FFN output 77 / 71; 4096 rows: 18.1 / 19.7, 16.2 /
+#     18.2, 24.5 / 37.6, 29.7 / 30.3; 512 rows: 7.5 / 8.7, 9.2 / 11.2, 8.8 / 13.6, 13.6 /
+#     15.9; 64 rows: 5.4 / 7.6, 7.2 / 9.2, 5.6 / 10.5, 8.9 / 11.1;
+#   * an F.linear call also costs about 19 us of hipBLASLt host time against a few.
+# torch.compile traces hip_gemm_rows's rule instead: below HIP_GEMM_MIN_ROWS rows F.linear,
+# which Inductor fuses.  Checked on every call: the layer program binds the fused steps once
+# per bucket, while B varies per call.
 HIP_GEMM_MIN_ROWS = 16384
 HIP_GEMM_EAGER_MAX_ROWS = 2048
 HIP_GEMM_EAGER_MAX_WIDTH = 768
@@ -141,8 +133,9 @@ def eager_small_gemm(x: torch.Tensor, n: int) -> bool:
 
 def hip_gemm_rows(x: torch.Tensor, n: int | None = None) -> bool:
     """The rule by rows and launch mode for the projection of ``x`` (``[..., K]``) to
-    ``n`` columns (default K): True from :data:`HIP_GEMM_MIN_ROWS` rows and in
-    launch-bound eager forwards (:func:`eager_small_gemm`)."""
+    ``n`` columns (default K) that ``torch.compile`` traces: True from
+    :data:`HIP_GEMM_MIN_ROWS` rows, and outside tracing in launch-bound eager forwards
+    (:func:`eager_small_gemm`)."""
 
     k = x.shape[-1]
     if k <= 0 or x.device.type != "cuda":
@@ -156,13 +149,9 @@ def projection_on_hip(x: torch.Tensor, n: int) -> bool:
     """True if the projection of ``x`` (``[..., K]``) to ``n`` columns runs on the
     hand-written GEMM (see the rules above)."""
 
-    k = x.shape[-1]
-    if k <= 0 or x.device.type != "cuda":
-        return False
-    if not torch.compiler.is_compiling() and (
-            k < 3 * n or x.numel() // k >= HIP_GEMM_LONG_K_ROWS):
-        return True
-    return hip_gemm_rows(x, n)
+    if torch.compiler.is_compiling():
+        return hip_gemm_rows(x, n)
+    return x.shape[-1] > 0 and x.device.type == "cuda"
 
 
 # Tile configuration the encoder asks dflash_linear_fwd for (bits 8.. of its
@@ -216,6 +205,39 @@ def linear_epilogue(
 
 @linear_epilogue.register_fake
 def _linear_epilogue_fake(x, weight, bias, residual, epilogue):
+    return x.new_empty(x.shape[:-1] + (weight.shape[0],))
+
+
+@_lib.hip_op("disentangled_flash::linear_add_layernorm")
+def linear_add_layernorm(
+    x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, residual: torch.Tensor,
+    norm_weight: torch.Tensor, norm_bias: torch.Tensor, eps: float
+) -> torch.Tensor:
+    """``LayerNorm(x @ weight.T + bias + residual)``: the hand-written GEMM, then the fused
+    add + LayerNorm, which for few rows also adds the GEMM's K ranges."""
+
+    lib = _lib.load()
+    k = x.shape[-1]
+    n = weight.shape[0]
+    rows = x.numel() // k if k else 0
+    if residual.shape[-1] != n or residual.numel() != rows * n or residual.dtype != x.dtype \
+            or residual.device != x.device or not residual.is_contiguous():
+        raise ValueError("linear_add_layernorm: residual must be contiguous [..., N] of the "
+                         "input's rows, dtype and device")
+    out = x.new_empty(x.shape[:-1] + (n,))
+    size = lib.dflash_output_block_workspace_bytes(rows, n, k)
+    workspace = torch.empty(size, device=x.device, dtype=torch.uint8)
+    code = lib.dflash_output_block_fwd(
+        x.data_ptr(), weight.data_ptr(), bias.data_ptr(), residual.data_ptr(),
+        norm_weight.data_ptr(), norm_bias.data_ptr(), out.data_ptr(), rows, n, k, float(eps),
+        _lib.DTYPE_CODES[x.dtype], workspace.data_ptr(), size,
+        _lib.current_stream_handle(x.device))
+    _lib.check(code, "dflash_output_block_fwd")
+    return out
+
+
+@linear_add_layernorm.register_fake
+def _linear_add_layernorm_fake(x, weight, bias, residual, norm_weight, norm_bias, eps):
     return x.new_empty(x.shape[:-1] + (weight.shape[0],))
 
 
@@ -318,10 +340,9 @@ def output_block(module: nn.Module, hidden_states: torch.Tensor,
     norm = module.LayerNorm
     if linear_fits(dense) and hidden_states.dtype == dense.weight.dtype \
             and projection_on_hip(hidden_states, dense.out_features):
-        projected = linear_epilogue(gemm_rows(hidden_states), dense.weight, dense.bias, None,
-                                    GEMM_BIAS)
-    else:
-        projected = F.linear(hidden_states, dense.weight, dense.bias)
+        return linear_add_layernorm(gemm_rows(hidden_states), dense.weight, dense.bias, residual,
+                                    norm.weight, norm.bias, norm.eps)
+    projected = F.linear(hidden_states, dense.weight, dense.bias)
     return add_layernorm(projected, residual, norm.weight, norm.bias, norm.eps)
 
 

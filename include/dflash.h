@@ -287,6 +287,22 @@ DFLASH_API int dflash_linear_fwd(const void* x, const void* weight, const void* 
                                  const void* residual, void* y, int M, int N, int K,
                                  int epilogue, int dtype, void* stream);
 
+/*
+ * An output block of an encoder layer: out = LayerNorm(T(T(x.W^T + bias) + residual)),
+ * DebertaV2SelfOutput / DebertaV2Output (_reference.py:108-112, 482-485): the projection
+ * of dflash_linear_fwd (x [M, K], weight [N, K], fp16 or bf16, its shape and alignment
+ * rules) and the kernel of dflash_add_layernorm_fwd (residual, out [M, N]; gamma, beta
+ * [N]; N at most 4096).  With few rows the projection's K is split over workgroups
+ * and the LayerNorm adds the fp32 partial sums.  residual must not be NULL.
+ *   workspace : at least dflash_output_block_workspace_bytes(M, N, K) bytes, 16-byte
+ *               aligned; its contents need not outlive the kernels.
+ */
+DFLASH_API size_t dflash_output_block_workspace_bytes(int M, int N, int K);
+DFLASH_API int dflash_output_block_fwd(const void* x, const void* weight, const void* bias,
+                                       const void* residual, const void* gamma, const void* beta,
+                                       void* out, int M, int N, int K, float eps, int dtype,
+                                       void* workspace, size_t workspace_bytes, void* stream);
+
 /* Text for a return code of any dflash_* entry point. */
 DFLASH_API const char* dflash_error_string(int code);
 
