@@ -32,6 +32,19 @@ _c_int = ctypes.c_int
 _c_int64 = ctypes.c_int64
 _c_float = ctypes.c_float
 
+
+class EncoderLayer(ctypes.Structure):
+    """``dflash_encoder_layer``: the pointers and sizes of one layer."""
+
+    _fields_ = [(name, _c_void_p) for name in (
+        "qkv_weight", "qkv_bias", "pos_key", "pos_query", "delta_to_local",
+        "attention_weight", "attention_bias", "attention_gamma", "attention_beta",
+        "inner_weight", "inner_bias",
+        "output_weight", "output_bias", "output_gamma", "output_beta")] + [
+        (name, _c_float) for name in ("score_scale_log2", "attention_eps", "output_eps")] + [
+        (name, _c_int) for name in ("heads", "head_dim", "slots", "hidden", "inner", "dtype")]
+
+
 _handle: ctypes.CDLL | None = None
 _load_error: str | None = None
 
@@ -109,6 +122,15 @@ def _bind(lib: ctypes.CDLL) -> None:
         _c_int, _c_int, _c_int, _c_float, _c_int,                # M, N, K, eps, dtype
         _c_void_p, ctypes.c_size_t, _c_void_p,                   # workspace, bytes, stream
     ]
+    lib.dflash_encoder_layer_workspace_bytes.restype = ctypes.c_size_t
+    lib.dflash_encoder_layer_workspace_bytes.argtypes = [
+        ctypes.POINTER(EncoderLayer), _c_int, _c_int]            # layer, B, L
+    lib.dflash_encoder_layer_fwd.restype = _c_int
+    lib.dflash_encoder_layer_fwd.argtypes = [
+        ctypes.POINTER(EncoderLayer), _c_void_p, _c_void_p, _c_void_p,  # layer, x, mask, out
+        _c_int, _c_int,                                          # B, L
+        _c_void_p, ctypes.c_size_t, _c_void_p,                   # workspace, bytes, stream
+    ]
     lib.dflash_error_string.restype = ctypes.c_char_p
     lib.dflash_error_string.argtypes = [_c_int]
     lib.dflash_abi_version.restype = _c_int
@@ -172,6 +194,14 @@ def current_stream_handle(device: torch.device) -> int:
     if _raw_stream is not None:
         return _raw_stream(device.index if device.index is not None else torch.cuda.current_device())
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def runs_directly(tensor: torch.Tensor) -> bool:
+    """True outside tracing (torch.compile, export) and dispatch modes, for a plain CUDA
+    tensor: the library may be called on its address."""
+
+    return (type(tensor) in _PLAIN_TENSORS and tensor.device.type == "cuda"
+            and not torch.compiler.is_compiling() and _get_dispatch_mode() is None)
 
 
 def hip_op(name: str):

@@ -241,6 +241,12 @@ def _linear_add_layernorm_fake(x, weight, bias, residual, norm_weight, norm_bias
     return x.new_empty(x.shape[:-1] + (weight.shape[0],))
 
 
+def gemm_width_fits(n: int, k: int) -> bool:
+    """True if the hand-written GEMM takes an ``[N, K]`` weight."""
+
+    return (n % 128 == 0 or n % 192 == 0) and k % 32 == 0
+
+
 def gemm_fits(weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
     """True if ``F.linear(x, weight, bias)`` can run on :func:`linear_epilogue`.
 
@@ -256,7 +262,7 @@ def gemm_fits(weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
         return False
     if not weight.is_contiguous() or weight.device.type != "cuda":
         return False
-    return (n % 128 == 0 or n % 192 == 0) and k % 32 == 0
+    return gemm_width_fits(n, k)
 
 
 def linear_fits(linear: nn.Module) -> bool:

@@ -303,6 +303,37 @@ DFLASH_API int dflash_output_block_fwd(const void* x, const void* weight, const 
                                        void* out, int M, int N, int K, float eps, int dtype,
                                        void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * One encoder layer (DebertaV2Layer, _reference.py:488-516, as run by
+ * DebertaV2InferenceEncoder.forward_prepared, deberta.py:262-276): QKV projection
+ * (dflash_linear_fwd), attention (dflash_attention_rel_fwd_split, split as planned), the
+ * attention's output block, the FFN intermediate with its erf GELU and the FFN's
+ * output block (dflash_output_block_fwd), launched one after the other.
+ *   x, out    : [B, L, hidden] contiguous, fp16 or bf16; mask uint8 [B, L]
+ *   workspace : at least dflash_encoder_layer_workspace_bytes(layer, B, L) bytes,
+ *               16-byte aligned (0: arguments the call refuses)
+ * The weights are nn.Linear's [out, in]; the rules of the calls above hold for each.
+ * An argument that only a later call refuses leaves the earlier ones launched.
+ */
+typedef struct dflash_encoder_layer {
+  const void *qkv_weight, *qkv_bias;                 /* [3*heads*head_dim, hidden] */
+  const void *pos_key, *pos_query;                   /* [heads, slots, head_dim]; NULL: mode off */
+  const int32_t* delta_to_local;                     /* [2L-1] */
+  const void *attention_weight, *attention_bias;     /* [hidden, heads*head_dim] */
+  const void *attention_gamma, *attention_beta;      /* [hidden] */
+  const void *inner_weight, *inner_bias;             /* [inner, hidden] */
+  const void *output_weight, *output_bias;           /* [hidden, inner] */
+  const void *output_gamma, *output_beta;            /* [hidden] */
+  float score_scale_log2, attention_eps, output_eps;
+  int heads, head_dim, slots, hidden, inner, dtype;
+} dflash_encoder_layer;
+
+DFLASH_API size_t dflash_encoder_layer_workspace_bytes(const dflash_encoder_layer* layer, int B,
+                                                       int L);
+DFLASH_API int dflash_encoder_layer_fwd(const dflash_encoder_layer* layer, const void* x,
+                                        const uint8_t* mask, void* out, int B, int L,
+                                        void* workspace, size_t workspace_bytes, void* stream);
+
 /* Text for a return code of any dflash_* entry point. */
 DFLASH_API const char* dflash_error_string(int code);
 
