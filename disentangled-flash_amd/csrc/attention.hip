@@ -188,7 +188,8 @@ int rel_forward(const void* query, const void* key, const void* value, int64_t s
   rp.has_c2p = has_c2p;
   rp.has_p2c = has_p2c;
   rp.splits = 1;
-  rp.qw = rel_attention_qw(B, H, L, D, current_device_cus(), has_c2p != 0);
+  rp.cus = current_device_cus();
+  rp.qw = rel_attention_qw(B, H, L, D, rp.cus, has_c2p != 0);
   rp.fast = dtype == DFLASH_DTYPE_FP32 && !strict_fp32;
   if (splits > 1 && dtype != DFLASH_DTYPE_FP32) {  // fp32 runs unsplit
     if (splits > 8) return DFLASH_ERR_SHAPE;

@@ -41,6 +41,8 @@ struct RelParams {
   // last slice, b = B - 1 and h = H - 1, may run as a launch of its own); 0
   // otherwise.
   int bh0;
+  int cus;        // CUs of the device
+  int by_length;  // 1 = the longest sequences of the batch first, set by the launcher
 };
 
 // fp16 / bf16 / fp32, D in {32, 64, 128}; arguments already validated by the

@@ -387,6 +387,47 @@ struct RelLayout {
   static constexpr size_t bytes = cw_off + size_t(kWaves) * QW * CW_LD * sizeof(T);
 };
 
+// The batch index of place `place` when the sequences are put in order of falling
+// length, kSortBatch sequences at a time; every wavefront finds the same order.  A
+// length is taken as the kept keys among four probes of the mask (5/8, 6/8, 7/8 and
+// the end of L), one byte per lane and one load in all: with eight probes a lane the
+// order cost 1.2 us a workgroup.  A mask with holes only makes the order worse; it is
+// a permutation for any mask.
+// Probe and order are two steps so that loads of other things go out in between.
+constexpr int kSortBatch = 16;
+// Built for the forms of one workgroup per CU (fp32, and 16-bit d = 128 on the 32-row
+// tile), whose workgroups are the long ones.  With two per CU a CU evens them out by
+// itself: d = 64 ragged 52.2 -> 51.5 us but full 87.4 -> 88.9, d = 32 full 27.8 -> 28.7.
+template <int WGS, bool SPLIT, bool TABLE>
+constexpr bool rel_by_length() {
+  return WGS == 1 && !SPLIT && !TABLE;
+}
+__device__ inline uint8_t length_probe(const uint8_t* mask, int B, int L, int place) {
+  const int lane = threadIdx.x & 63;
+  const int first = place & ~(kSortBatch - 1);
+  const int row = min(lane >> 2, min(B - first, kSortBatch) - 1);
+  const int key = (L * ((lane & 3) + 5) >> 3) - 1;
+  return mask[static_cast<int64_t>(first + row) * L + max(key, 0)];
+}
+__device__ inline int sequence_by_length(uint8_t probe, int B, int place) {
+  const int lane = threadIdx.x & 63;
+  const int first = place & ~(kSortBatch - 1);
+  const int count = min(B - first, kSortBatch);
+  const uint64_t kept = __ballot(probe != 0);
+  const bool valid = lane < count;
+  const int n = valid ? __popc(static_cast<uint32_t>(kept >> (4 * lane & 63)) & 15u) : -1;
+  int before = 0;  // sequences longer than the present length
+  int at = -1;     // place of this lane's sequence
+#pragma unroll
+  for (int v = 4; v >= 0; --v) {
+    const uint32_t same = static_cast<uint32_t>(__ballot(n == v));
+    const int rank = __builtin_amdgcn_mbcnt_lo(same, static_cast<uint32_t>(before));
+    if (n == v) at = rank;
+    before += __popc(same);
+  }
+  return first + __builtin_ctz(static_cast<uint32_t>(__ballot(valid && at == place - first)));
+}
+
 }  // namespace
 
 template <typename T, int D, int QW, int BN, int VBUFS, int WGS, bool C2P, bool P2C, bool SPLIT,
@@ -454,31 +495,62 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
   const int g = lane >> 4;
 
   const int L = p.L;
-  const int mk = xcd_logical_block(blockIdx.x, gridDim.x);
-  // Key split of the split-key form (the splits of a block are neighbours).
-  const int split = SPLIT ? mk % p.splits : 0;
-  const int m = SPLIT ? mk / p.splits : mk;
-  const int qblk = m % p.nqb;
-  // Groups of query blocks in head-major order (the batch index fastest):
-  // each XCD's contiguous range of groups then holds sequences of every
-  // length of the batch, not a few neighbouring ones, so the XCDs finish
-  // together on ragged batches (C5 valid-length cycle: d = 128 71.8 -> 53.1
-  // us, d = 32 28.3 -> 21.5 us; unpadded unchanged).  A group's query blocks
-  // stay on one XCD.  The last group is the last (b, h) slice either way.
-  const int bh = p.bh0 + m / p.nqb;
-  const int h = bh / p.B;
-  const int b = bh - h * p.B;
+  int split = 0, qblk, b, h;
+  constexpr bool kByLength = rel_by_length<WGS, SPLIT, TABLE>();
+  bool by_length = false;
+  uint8_t length = 0;
+  if constexpr (kByLength) by_length = p.by_length != 0;
+  if (by_length) {
+    // Groups dealt to the XCDs in turn (the last groups % 8 split by block), the
+    // longest sequences of the batch first.
+    const int groups = p.B * p.H;
+    const int per = groups / 8;
+    const int n = blockIdx.x;
+    int group;
+    if (n < 8 * per * p.nqb) {
+      const int idx = n / 8;
+      group = idx / p.nqb * 8 + n % 8;
+      qblk = idx % p.nqb;
+    } else {
+      const int l = xcd_logical_block(n - 8 * per * p.nqb, (groups - 8 * per) * p.nqb);
+      group = 8 * per + l / p.nqb;
+      qblk = l % p.nqb;
+    }
+    const int place = group / p.H;  // of the sequence, by length
+    h = group - place * p.H;
+    b = place;
+    length = length_probe(p.mask, p.B, L, place);
+  } else {
+    const int mk = xcd_logical_block(blockIdx.x, gridDim.x);
+    // Key split of the split-key form (the splits of a block are neighbours).
+    split = SPLIT ? mk % p.splits : 0;
+    const int m = SPLIT ? mk / p.splits : mk;
+    qblk = m % p.nqb;
+    // Groups of query blocks in head-major order (the batch index fastest):
+    // each XCD's contiguous range of groups then holds sequences of every
+    // length of the batch, not a few neighbouring ones, so the XCDs finish
+    // together on ragged batches (C5 valid-length cycle: d = 128 71.8 -> 53.1
+    // us, d = 32 28.3 -> 21.5 us; unpadded unchanged).  A group's query blocks
+    // stay on one XCD.  The last group is the last (b, h) slice either way.
+    const int bh = p.bh0 + m / p.nqb;
+    h = bh / p.B;
+    b = bh - h * p.B;
+  }
   const int i0 = qblk * BM;
   const int i0w = i0 + wave * QW;
   const uint32_t sl_bytes = static_cast<uint32_t>(p.sl) * ES;
 
   // Buffer resources.  Rows past L read as zero; the bound is the end of row L-1.
-  const uint32_t head_bytes = (static_cast<uint32_t>(L - 1) * static_cast<uint32_t>(p.sl) + D) * ES;
-  const int64_t head_off = static_cast<int64_t>(b) * p.sb + static_cast<int64_t>(h) * p.sh;
-  const auto rq = make_rsrc(reinterpret_cast<const T*>(p.q) + head_off, head_bytes);
-  const auto rk = make_rsrc(reinterpret_cast<const T*>(p.k) + head_off, head_bytes);
-  const auto rv = make_rsrc(reinterpret_cast<const T*>(p.v) + head_off, head_bytes);
-  const auto rmask = make_rsrc(p.mask + static_cast<int64_t>(b) * L, static_cast<uint32_t>(L));
+  __amdgpu_buffer_rsrc_t rq, rk, rv, rmask;
+  auto set_sequence = [&]() {
+    const uint32_t head_bytes = (static_cast<uint32_t>(L - 1) * static_cast<uint32_t>(p.sl) + D) * ES;
+    const int64_t head_off = static_cast<int64_t>(b) * p.sb + static_cast<int64_t>(h) * p.sh;
+    rq = make_rsrc(reinterpret_cast<const T*>(p.q) + head_off, head_bytes);
+    rk = make_rsrc(reinterpret_cast<const T*>(p.k) + head_off, head_bytes);
+    rv = make_rsrc(reinterpret_cast<const T*>(p.v) + head_off, head_bytes);
+    rmask = make_rsrc(p.mask + static_cast<int64_t>(b) * L, static_cast<uint32_t>(L));
+  };
+  if constexpr (!kByLength) set_sequence();
   const uint32_t rel_bytes = static_cast<uint32_t>(p.S) * D * ES;
   const auto rkr = make_rsrc(reinterpret_cast<const T*>(p.pos_key) + static_cast<int64_t>(h) * p.S * D,
                              rel_bytes);
@@ -989,6 +1061,10 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
     for (int u = 0; u < PU; ++u) lp[u] = lut_load(lut_p_index(jstart, u));
     lutp = lut_load(lut_p_index(jstart + BN, 0));
   }
+  if constexpr (kByLength) {
+    if (by_length) b = sequence_by_length(length, p.B, b);
+    set_sequence();
+  }
   // Mask bytes: the first 512 of the sequence (for the extent), the
   // workgroup's queries and each lane's queries.  Bytes past L read as zero.
   uint8_t km[8];
@@ -1006,29 +1082,31 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
   // Workgroup and query flags from the mask bytes.
   bool wg_kept = false;
   bool wg_padded = false;
+  if constexpr (!kByLength) {
 #pragma unroll
-  for (int n = 0; n < kWgMaskLoads; ++n) {
-    const bool mine = 64 * n + lane < BM;
-    const bool kept = wm[n] != 0;
-    wg_kept = wg_kept || __any(kept);
-    wg_padded = wg_padded || __any(mine && i0 + 64 * n + lane < L && !kept);
-  }
-#pragma unroll
-  for (int qb = 0; qb < kQB; ++qb) qkept[qb] = qm[qb] != 0;
-
-  if (!wg_kept) {
-    if (SPLIT && split > 0) return;  // split 0 stores the mean of V
-    // Every query of the workgroup is padded (or past L): all rows are the mean of V.
-    v_mean();
-    const int row_lo = i0 + tid / (D / 4);
-    for (int i = row_lo; i < min(i0 + BM, L); i += kThreads / (D / 4)) {
-      const int d0 = 4 * (tid % (D / 4));
-      Quad<T> q;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) q[r] = static_cast<T>(vmean[d0 + r]);
-      *reinterpret_cast<Quad<T>*>(outp + (static_cast<int64_t>(b) * L + i) * row_stride + h * D + d0) = q;
+    for (int n = 0; n < kWgMaskLoads; ++n) {
+      const bool mine = 64 * n + lane < BM;
+      const bool kept = wm[n] != 0;
+      wg_kept = wg_kept || __any(kept);
+      wg_padded = wg_padded || __any(mine && i0 + 64 * n + lane < L && !kept);
     }
-    return;
+#pragma unroll
+    for (int qb = 0; qb < kQB; ++qb) qkept[qb] = qm[qb] != 0;
+
+    if (!wg_kept) {
+      if (SPLIT && split > 0) return;  // split 0 stores the mean of V
+      // Every query of the workgroup is padded (or past L): all rows are the mean of V.
+      v_mean();
+      const int row_lo = i0 + tid / (D / 4);
+      for (int i = row_lo; i < min(i0 + BM, L); i += kThreads / (D / 4)) {
+        const int d0 = 4 * (tid % (D / 4));
+        Quad<T> q;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) q[r] = static_cast<T>(vmean[d0 + r]);
+        *reinterpret_cast<Quad<T>*>(outp + (static_cast<int64_t>(b) * L + i) * row_stride + h * D + d0) = q;
+      }
+      return;
+    }
   }
 
   // Rows of the tile-0 windows, then Q and the K/V of tile 0 (a workgroup
@@ -1070,6 +1148,34 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
   } else {
     prefetch_k(jstart);
     prefetch_v(jstart);
+  }
+  // By length, the mask bytes came a load later than the lookups, and the loads above
+  // went out without waiting for them (d = 128 ragged 66.1 against 66.7 us waiting).
+  if constexpr (kByLength) {
+#pragma unroll
+    for (int n = 0; n < kWgMaskLoads; ++n) {
+      const bool mine = 64 * n + lane < BM;
+      const bool kept = wm[n] != 0;
+      wg_kept = wg_kept || __any(kept);
+      wg_padded = wg_padded || __any(mine && i0 + 64 * n + lane < L && !kept);
+    }
+#pragma unroll
+    for (int qb = 0; qb < kQB; ++qb) qkept[qb] = qm[qb] != 0;
+
+    if (!wg_kept) {
+      if constexpr (kDirect) wait_vmem<0>();  // the copies land before LDS is reused
+      // Every query of the workgroup is padded (or past L): all rows are the mean of V.
+      v_mean();
+      const int row_lo = i0 + tid / (D / 4);
+      for (int i = row_lo; i < min(i0 + BM, L); i += kThreads / (D / 4)) {
+        const int d0 = 4 * (tid % (D / 4));
+        Quad<T> q;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) q[r] = static_cast<T>(vmean[d0 + r]);
+        *reinterpret_cast<Quad<T>*>(outp + (static_cast<int64_t>(b) * L + i) * row_stride + h * D + d0) = q;
+      }
+      return;
+    }
   }
   // Tile 1 (d = 64 only: d = 128 has no registers to spare here, and d = 32,
   // whose tiles are short, measured faster without it): K/V and the rows of
@@ -1810,6 +1916,13 @@ int launch_rel(const RelParams& base, hipStream_t stream) {
                        rel_kv_planes3<T, D, FAST, C2P>()>;
   RelParams prm = base;
   prm.nqb = (prm.L + LY::BM - 1) / LY::BM;
+  // Longest sequences first where the grid runs in more than one round: the last round
+  // then holds the short ones (fp32 d = 64, H = 12, L = 384, B = 8 ragged 91.1 -> 77.5
+  // us; B = 30, L = 300, H = 6 95.2 -> 89.4; d = 128, H = 8, L = 512, B = 16 ragged 71.3
+  // -> 66.1).  With every sequence full it buys nothing and costs under 1 us a launch
+  // (fp32 107.0 -> 108.6, d = 128 72.1 -> 72.4).  A single round starts all at once.
+  prm.by_length = rel_by_length<WGS, false, TABLE>() && prm.B > 1 && prm.splits <= 1 &&
+                  static_cast<int64_t>(prm.nqb) * prm.B * prm.H > prm.cus;
   // The split-key form exists for the default 16-bit tile (QW = 32 at d <= 64,
   // 16 at d = 128); fp32 never splits.
   constexpr bool kSplitBuilt = sizeof(T) == 2 && (D >= 128 ? QW == 16 : QW == 32) && !TABLE;
