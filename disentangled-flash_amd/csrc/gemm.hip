@@ -68,33 +68,17 @@
 
 #include "device_common.h"
 #include "dflash.h"
+#include "gemm_tile.h"
 #include "layernorm.h"
 
 namespace dflash {
 
 namespace {
 
-constexpr int kStepK = 32;           // k of one MFMA step
-constexpr int kSlabK = 2 * kStepK;    // k of one slab (128-byte rows)
-
 constexpr int kEpiBias = 0;
 constexpr int kEpiBiasGelu = 1;
 constexpr int kEpiBiasAdd = 2;
 constexpr int kEpiPartial = 3;  // fp32 sums of one of `splits` ranges of K, no bias
-
-// Chunk permutation of slab row r: 16-byte chunk k of the row sits at position
-// k ^ slab_swizzle(r).  Eight consecutive rows hit eight different chunks of a
-// 128-byte window, and of sixteen no two the same chunk of a 256-byte one.
-// Depends on r mod 16 only.
-__device__ constexpr int slab_swizzle(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
-// Output column (inside the tile) of W row r of a slab: row x = 4a + b of the
-// 16-row blocks 2i and 2i + 1 holds columns 32i + 8a + b and 32i + 8a + 4 + b.
-__device__ constexpr int w_row(int r) {
-  const int block = r >> 4;
-  const int x = r & 15;
-  return 8 * (x >> 2) + (x & 3) + 4 * (block & 1) + 32 * (block >> 1);
-}
 
 // GELU in its erf form, x Phi(x), with Phi(-a) = 2^P(a) for a = |x|: P is a
 // polynomial of degree 8 fitted to log2 Phi(-a) on [0, 6] (minimax weighted with
@@ -119,20 +103,19 @@ __device__ inline float gelu_erf(float x) {
   return x * (x >= 0.0f ? 1.0f - tail : tail);
 }
 
-// One buffer_load_dwordx4 with the LDS bit: 16 bytes per lane from `off` + `koff`
-// (`koff` uniform and not range-checked; rows past the tile's last have `off` past
-// the resource's size and store zeros) to LDS at `lds` + 16 * lane (`lds` uniform,
-// in M0; one wait state between the write of M0 and the load).  Inline assembly,
-// so that the compiler does not wait for copies in flight before fragment reads;
+// One buffer_load_dwordx4 with the LDS bit: 16 bytes per lane from `off` + `scalar`
+// (`scalar` uniform; zeros where `off` is past the resource's size) to LDS at `lds` + 16 *
+// lane (`lds` uniform, in M0; one wait state between the write of M0 and the load).  Inline
+// assembly, so that the compiler does not wait for copies in flight before fragment reads;
 // they are awaited by wait_vmem and the slab's barrier.
-__device__ inline void copy16_to_lds(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t koff,
+__device__ inline void copy16_to_lds(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t scalar,
                                      uint32_t lds) {
   asm volatile(
       "s_mov_b32 m0, %0\n\t"
       "s_nop 0\n\t"
       "buffer_load_dwordx4 %1, %2, %3 offen lds"
       :
-      : "s"(lds), "v"(off), "s"(r), "s"(koff)
+      : "s"(lds), "v"(off), "s"(r), "s"(scalar)
       : "memory");
 }
 
@@ -167,35 +150,6 @@ __device__ inline void wait_vmem() {
 
 }  // namespace
 
-// Tile configuration: a workgroup of WAVES_M x WAVES_N wavefronts computes a
-// BM x BN tile of Y (wavefront tile BM/WAVES_M x BN/WAVES_N) through a ring of
-// STAGES slabs; WGS workgroups per CU are budgeted for.
-template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int WGS_, int STAGES_ = 2>
-struct GemmConfig {
-  static constexpr int BM = BM_;
-  static constexpr int BN = BN_;
-  static constexpr int WAVES_M = WAVES_M_;
-  static constexpr int WAVES_N = WAVES_N_;
-  static constexpr int WGS = WGS_;
-  static constexpr int STAGES = STAGES_;
-  static constexpr int WAVES = WAVES_M * WAVES_N;
-  static constexpr int THREADS = 64 * WAVES;
-  static constexpr int WM = BM / WAVES_M;
-  static constexpr int WN = BN / WAVES_N;
-  static constexpr int MB = WM / 16;            // 16-row blocks per wavefront
-  static constexpr int NB = WN / 16;            // 16-column blocks per wavefront
-  static constexpr int A_LOADS = BM / 8 / WAVES;  // copies (8 rows each) per wavefront and slab
-  static constexpr int B_LOADS = BN / 8 / WAVES;
-  static constexpr int LOADS = A_LOADS + B_LOADS;
-  static constexpr int A_BYTES = BM * kSlabK * 2;
-  static constexpr int SLAB = (BM + BN) * kSlabK * 2;
-  static constexpr int LDS = STAGES * SLAB;
-  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "copies split evenly");
-  static_assert(WM % 16 == 0 && WN % 32 == 0, "whole MFMA blocks, column blocks in pairs");
-  static_assert(STAGES >= 2 && LDS * WGS <= 160 * 1024, "LDS of a CU");
-  static_assert((STAGES - 1) * LOADS <= 63, "vmcnt range");
-};
-
 struct GemmArgs {
   const void* x;
   const void* w;
@@ -209,8 +163,7 @@ struct GemmArgs {
   int xcds_m;  // XCDs along the rows (1, 2, 4, 8); 8 / xcds_m along the columns
 };
 
-// FAR: 64-bit copy addresses (tile rows past 32-bit byte offsets).
-template <typename T, int EPI, typename CF, bool FAR = false>
+template <typename T, int EPI, typename CF, Copies COPIES>
 __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) {
   using M = Mma<T>;
   using F = typename M::frag;
@@ -246,54 +199,52 @@ __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) 
   const int m_base = mb * CF::BM;
   const int n_base = nb * CF::BN;
   const int ld = a.K;  // row stride of X and W
-  const int all_slabs = (a.K + kSlabK - 1) / kSlabK;  // (the last may be half: K % 32 == 0)
-  const int slab_lo = EPI == kEpiPartial ? all_slabs * split / a.splits : 0;
-  const int KT = EPI == kEpiPartial ? all_slabs * (split + 1) / a.splits - slab_lo : all_slabs;
-  const int K = min(a.K - slab_lo * kSlabK, KT * kSlabK);  // of this workgroup
+  const KRange range = k_range(a.K, split, EPI == kEpiPartial ? a.splits : 1);
+  const int KT = range.slabs;
+  const int K = range.k;  // of this workgroup
   const uint32_t row_bytes = static_cast<uint32_t>(ld) * 2u;
   const int rows = min(CF::BM, a.M - m_base);
-  const T* X = reinterpret_cast<const T*>(a.x) + static_cast<int64_t>(m_base) * ld + slab_lo * kSlabK;
-  const T* W = reinterpret_cast<const T*>(a.w) + static_cast<int64_t>(n_base) * ld + slab_lo * kSlabK;
-  const uint32_t skipped = static_cast<uint32_t>(slab_lo) * (kSlabK * 2);
-  const uint32_t x_bytes = static_cast<uint32_t>(rows) * row_bytes - skipped;
-  const uint32_t w_bytes = static_cast<uint32_t>(CF::BN) * row_bytes - skipped;
+  const T* X = reinterpret_cast<const T*>(a.x) + static_cast<int64_t>(m_base) * ld + range.first * kSlabK;
+  const T* W = reinterpret_cast<const T*>(a.w) + static_cast<int64_t>(n_base) * ld + range.first * kSlabK;
+  const uint32_t x_bytes = tile_bytes(rows, row_bytes, range);
+  const uint32_t w_bytes = tile_bytes(CF::BN, row_bytes, range);
 
-  // Copy j of a slab fetches eight slab rows (8 lanes a row): row and source
-  // chunk of this lane, and its byte offset from the tile's first row.
-  auto slab_row = [&](int j) { return (j * CF::WAVES + wave) * 8 + (lane >> 3); };
-  auto chunk_of = [&](int r) { return (lane & 7) ^ slab_swizzle(r); };
+  // Byte offset of this lane's 16 bytes of copy j from the tile's first row.
   uint32_t xoff[CF::A_LOADS], woff[CF::B_LOADS];
 #pragma unroll
-  for (int j = 0; j < CF::A_LOADS; ++j)
-    xoff[j] = static_cast<uint32_t>(slab_row(j)) * row_bytes + chunk_of(slab_row(j)) * 16;
+  for (int j = 0; j < CF::A_LOADS; ++j) {
+    const int r = copy_row<CF>(j, wave, lane);
+    xoff[j] = static_cast<uint32_t>(r) * row_bytes + copy_chunk(r, lane) * 16;
+  }
 #pragma unroll
-  for (int j = 0; j < CF::B_LOADS; ++j)
-    woff[j] = static_cast<uint32_t>(w_row(slab_row(j))) * row_bytes + chunk_of(slab_row(j)) * 16;
+  for (int j = 0; j < CF::B_LOADS; ++j) {
+    const int r = copy_row<CF>(j, wave, lane);
+    woff[j] = static_cast<uint32_t>(w_row(r)) * row_bytes + copy_chunk(r, lane) * 16;
+  }
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
   // The k order starts at a slab of its own on each XCD and wraps around.
   const int k0 = K % kSlabK == 0 ? ((p & 7) * KT) >> 3 : 0;
-  auto slab_at = [&](int kt) { return kt + k0 < KT ? kt + k0 : kt + k0 - KT; };
   // Copy j of slab `kt` into ring stage `stage`.  Past the last slab it fetches
-  // nothing (a resource of size 0: zeros into a stage that is not read again),
-  // so that every slab issues the same number of copies and the waits are
-  // compile-time.
+  // nothing (zeros into a stage that is not read again), so that every slab issues
+  // the same number of copies and the waits are compile-time.
   auto copy = [&](int j, int kt, uint32_t stage) {
     const bool is_x = j < CF::A_LOADS;
     const int jj = is_x ? j : j - CF::A_LOADS;
     const uint32_t dst = __builtin_amdgcn_readfirstlane(
         lds0 + stage * CF::SLAB + (is_x ? 0 : CF::A_BYTES) + (jj * CF::WAVES + wave) * 1024);
-    if constexpr (FAR) {
-      // Rows past M repeat row M - 1; slabs and chunks past K repeat k 0 .. 31 of the
-      // last 32 (their products are not computed).
-      const int r = is_x ? min(slab_row(jj), rows - 1) : w_row(slab_row(jj));
-      const int k = min(slab_at(min(kt, KT - 1)) * kSlabK + chunk_of(slab_row(jj)) * 8, K - 8);
-      copy16_to_lds_far((is_x ? X : W) + static_cast<int64_t>(r) * ld + k, dst);
+    if constexpr (COPIES == Copies::kFar) {
+      // Rows past M repeat row M - 1.
+      const int row = copy_row<CF>(jj, wave, lane);
+      const int r = is_x ? min(row, rows - 1) : w_row(row);
+      copy16_to_lds_far((is_x ? X : W) + static_cast<int64_t>(r) * ld +
+                            far_k(kt, k0, range, copy_chunk(row, lane)),
+                        dst);
     } else {
-      const uint32_t bytes = kt < KT ? (is_x ? x_bytes : w_bytes) : 0u;
+      const SlabCopy s = slab_copy<COPIES>(kt, k0, KT, is_x ? x_bytes : w_bytes,
+                                           is_x ? xoff[is_x ? jj : 0] : woff[is_x ? 0 : jj]);
       const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<T*>(is_x ? X : W), static_cast<short>(0), static_cast<int>(bytes), 0x00020000);
-      copy16_to_lds(rsrc, is_x ? xoff[is_x ? jj : 0] : woff[is_x ? 0 : jj],
-                    __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(slab_at(kt)) * (kSlabK * 2)), dst);
+          const_cast<T*>(is_x ? X : W), static_cast<short>(0), static_cast<int>(s.bytes), 0x00020000);
+      copy16_to_lds(rsrc, s.lane, __builtin_amdgcn_readfirstlane(s.scalar), dst);
     }
   };
 
@@ -438,21 +389,6 @@ __global__ __launch_bounds__(CF::THREADS, CF::WGS) void gemm_kernel(GemmArgs a) 
 
 namespace {
 
-// Tile configurations (columns a multiple of the tile's; rows ragged).  Large tiles need the
-// fewest bytes per product and fill the chip from about 256 tiles; small ones, with
-// deeper rings, give few rows more workgroups.  gemm_cost says which is chosen.
-using Cfg128x192 = GemmConfig<128, 192, 2, 2, 2>;
-using Cfg128x128 = GemmConfig<128, 128, 2, 2, 2>;
-using Cfg256x192 = GemmConfig<256, 192, 4, 2, 1>;
-using Cfg64x128 = GemmConfig<64, 128, 2, 2, 2, 3>;
-using Cfg64x64 = GemmConfig<64, 64, 2, 2, 4>;
-using Cfg256x256 = GemmConfig<256, 256, 4, 2, 1>;
-using Cfg128x192Deep = GemmConfig<128, 192, 4, 2, 1, 4>;
-using Cfg128x128Deep = GemmConfig<128, 128, 4, 2, 1, 5>;
-using Cfg128x64 = GemmConfig<128, 64, 4, 1, 2, 3>;
-using Cfg64x64Deep = GemmConfig<64, 64, 2, 2, 2, 5>;
-using Cfg32x64 = GemmConfig<32, 64, 2, 2, 2, 6>;
-
 // CUs of the current device (cached per device; 256 if it cannot be read).
 int gemm_device_cus() {
   static std::atomic<int> cache[64];
@@ -470,9 +406,9 @@ int gemm_device_cus() {
   return cus;
 }
 
-template <typename T, int EPI, typename CF, bool FAR = false>
-int launch_gemm(GemmArgs args, hipStream_t stream) {
-  constexpr auto* kernel = &gemm_kernel<T, EPI, CF, FAR>;
+template <typename T, int EPI, typename CF, Copies COPIES>
+int launch_copies(GemmArgs args, hipStream_t stream) {
+  constexpr auto* kernel = &gemm_kernel<T, EPI, CF, COPIES>;
   // The dynamic LDS limit is raised once per device (the attribute persists).
   static std::atomic<uint64_t> raised{0};
   int dev = 0;
@@ -518,6 +454,12 @@ int launch_gemm(GemmArgs args, hipStream_t stream) {
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(CF::THREADS), CF::LDS,
                      stream, args);
   return static_cast<int>(hipGetLastError());
+}
+
+template <typename T, int EPI, typename CF>
+int launch_gemm(const GemmArgs& args, hipStream_t stream) {
+  return args.K % kSlabK == 0 ? launch_copies<T, EPI, CF, Copies::kWhole>(args, stream)
+                              : launch_copies<T, EPI, CF, Copies::kHalf>(args, stream);
 }
 
 // Time of a launch in microseconds on a tile configuration, from its tiles and
@@ -590,7 +532,7 @@ int pick_config(const GemmArgs& args, int config, hipStream_t stream) {
   // A tile's rows must lie within 32-bit byte offsets of its first one (256 rows
   // of 2 K bytes); past that, 64 x 64 tiles with 64-bit copy addresses.
   if (args.K >= (1 << 23) && config >= 0 && config <= 11)
-    return launch_gemm<T, EPI, Cfg64x64, true>(args, stream);
+    return launch_copies<T, EPI, Cfg64x64, Copies::kFar>(args, stream);
   if (config == 0) {
     float us = 0.0f;
     config = best_config(args, EPI == kEpiBiasGelu, &us);
