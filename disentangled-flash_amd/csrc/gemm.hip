@@ -531,16 +531,18 @@ template <typename T, int EPI>
 int pick_config(const GemmArgs& args, int config, hipStream_t stream) {
   // A tile's rows must lie within 32-bit byte offsets of its first one (256 rows
   // of 2 K bytes); past that, 64 x 64 tiles with 64-bit copy addresses.
-  if (args.K >= (1 << 23) && config >= 0 && config <= 11)
-    return launch_copies<T, EPI, Cfg64x64, Copies::kFar>(args, stream);
+  const bool far = args.K >= (1 << 23);
+  if (config == 0 && far) config = 5;
   if (config == 0) {
     float us = 0.0f;
     config = best_config(args, EPI == kEpiBiasGelu, &us);
   }
   auto fits = [&](auto cf) { return args.N % decltype(cf)::BN == 0; };
-#define DFLASH_GEMM_CASE(NUM, CF) \
-  case NUM:                       \
-    return fits(CF{}) ? launch_gemm<T, EPI, CF>(args, stream) : DFLASH_ERR_SHAPE;
+#define DFLASH_GEMM_CASE(NUM, CF)                                                \
+  case NUM:                                                                      \
+    if (!fits(CF{})) return DFLASH_ERR_SHAPE;                                    \
+    if (far) return launch_copies<T, EPI, Cfg64x64, Copies::kFar>(args, stream); \
+    return launch_gemm<T, EPI, CF>(args, stream);
   switch (config) {
     DFLASH_GEMM_CASE(1, Cfg128x192)
     DFLASH_GEMM_CASE(2, Cfg128x128)

@@ -77,7 +77,9 @@ def test_rows_past_32_bit_offsets():
     b = torch.randn(64, generator=gen, device="cuda").half()
     r = torch.randn(3, 64, generator=gen, device="cuda").half()
     ref, lin, acc = _reference(x, w, b, r, 2, torch.float16)
-    for config in (0, 3, 11):
+    for config in (3, 12):  # columns that do not divide N, no configuration
+        assert _run(x, w, b, r, 2, config)[0] == -2
+    for config in (0, 10, 11):
         code, y = _run(x, w, b, r, 2, config)
         assert code == 0
         # fp32 accumulation over 2^18 MFMA steps one after the other: half a unit in the
