@@ -28,7 +28,7 @@ import torch
 from . import _lib
 from ._torch import TorchInferenceDisentangledSelfAttention
 from . import layers
-from .layers import GEMM_BIAS, gemm_fits, gemm_rows, linear_epilogue
+from .layers import GEMM_BIAS, gemm_rows, linear_epilogue
 from .modeling import DebertaAttentionConfig
 from .position import SharedPositionPlanCache
 
@@ -401,10 +401,7 @@ class HipInferenceDisentangledSelfAttention(TorchInferenceDisentangledSelfAttent
             raise RuntimeError(
                 "fused QKV projection is not prepared; call prepare_for_inference() first"
             )
-        if layers.USE_HIP_GEMM and hidden_states.device.type == "cuda" \
-                and layers.projection_on_hip(hidden_states, prep.qkv_weight.shape[0]) \
-                and gemm_fits(prep.qkv_weight, prep.qkv_bias) \
-                and hidden_states.dtype == prep.qkv_weight.dtype:
+        if layers.projection_on_hip(hidden_states, prep.qkv_weight, prep.qkv_bias):
             return linear_epilogue(gemm_rows(hidden_states), prep.qkv_weight, prep.qkv_bias, None,
                                    GEMM_BIAS)
         return super()._fused_projection(hidden_states)

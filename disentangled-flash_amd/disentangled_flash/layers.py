@@ -145,13 +145,24 @@ def hip_gemm_rows(x: torch.Tensor, n: int | None = None) -> bool:
     return eager_small_gemm(x, k if n is None else n)
 
 
-def projection_on_hip(x: torch.Tensor, n: int) -> bool:
-    """True if the projection of ``x`` (``[..., K]``) to ``n`` columns runs on the
-    hand-written GEMM (see the rules above)."""
+def projection_on_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
+    """True if ``F.linear(x, weight, bias)`` runs on the hand-written GEMM, by the rules
+    above and by the operands as they lie now (parameters may have been replaced since
+    the encoder was prepared); everything else stays on ``F.linear``."""
 
+    if not USE_HIP_GEMM or x.device.type != "cuda" or x.dim() == 0 \
+            or not gemm_fits(weight, bias) or x.dtype != weight.dtype \
+            or x.shape[-1] != weight.shape[1] or x.device != weight.device:
+        return False
     if torch.compiler.is_compiling():
-        return hip_gemm_rows(x, n)
-    return x.shape[-1] > 0 and x.device.type == "cuda"
+        return hip_gemm_rows(x, weight.shape[0])
+    n, k = weight.shape
+    if x.numel() // k * max(n, k) >= GEMM_MAX_ELEMENTS:
+        return False
+    # (x is copied where it lies askew, gemm_rows; without plain tensors there is no address
+    # to look at, and the op's dispatch decides.)
+    return not _lib.runs_directly(weight) \
+        or (weight.data_ptr() % 16 == 0 and bias.data_ptr() % 8 == 0)
 
 
 # Tile configuration the encoder asks dflash_linear_fwd for (bits 8.. of its
@@ -163,6 +174,7 @@ GEMM_BIAS = 0
 GEMM_BIAS_GELU = 1
 GEMM_BIAS_ADD = 2
 GEMM_DTYPES = (torch.float16, torch.bfloat16)
+GEMM_MAX_ELEMENTS = 1 << 31  # of x and of the output (dflash_linear_fwd takes fewer)
 
 
 @_lib.hip_op("disentangled_flash::linear_epilogue")
@@ -244,15 +256,15 @@ def _linear_add_layernorm_fake(x, weight, bias, residual, norm_weight, norm_bias
 def gemm_width_fits(n: int, k: int) -> bool:
     """True if the hand-written GEMM takes an ``[N, K]`` weight."""
 
-    return (n % 128 == 0 or n % 192 == 0) and k % 32 == 0
+    return n > 0 and (n % 128 == 0 or n % 192 == 0) and k > 0 and k % 32 == 0
 
 
 def gemm_fits(weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
     """True if ``F.linear(x, weight, bias)`` can run on :func:`linear_epilogue`.
 
-    That is: a bias, fp16 or bf16 weight and bias on a GPU, N a multiple of 128
-    or 192 (the tile widths) and K a multiple of 32 (the k-step) - every
-    projection of DeBERTa base, large and xlarge.
+    That is: fp16 or bf16 weight and bias on a GPU, contiguous, the bias of N elements, N
+    a multiple of 128 or 192 (the tile widths) and K a multiple of 32 (the k-step) -
+    every projection of DeBERTa base, large and xlarge.
     """
 
     if bias is None or weight.dim() != 2:
@@ -262,6 +274,9 @@ def gemm_fits(weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
         return False
     if not weight.is_contiguous() or weight.device.type != "cuda":
         return False
+    if bias.dim() != 1 or bias.shape[0] != n or not bias.is_contiguous() \
+            or bias.device != weight.device:
+        return False
     return gemm_width_fits(n, k)
 
 
@@ -270,9 +285,11 @@ def linear_fits(linear: nn.Module) -> bool:
 
 
 def gemm_rows(x: torch.Tensor) -> torch.Tensor:
-    """``x`` with dense rows (last dimension contiguous, rows packed)."""
+    """``x`` with dense rows (last dimension contiguous, rows packed) from a 16-byte boundary."""
 
-    return x if x.is_contiguous() else x.contiguous()
+    if not x.is_contiguous():
+        return x.contiguous()
+    return x.clone() if _lib.runs_directly(x) and x.data_ptr() % 16 else x
 
 
 def fusable_intermediate(module: nn.Module) -> bool:
@@ -298,10 +315,13 @@ def intermediate_block(module: nn.Module, hidden_states: torch.Tensor) -> torch.
     """``module(hidden_states)`` as one GEMM with the GELU in its epilogue, or the
     module itself where :func:`projection_on_hip` says so."""
 
-    if not projection_on_hip(hidden_states, module.dense.out_features):
+    dense = module.dense
+    if not isinstance(dense, nn.Linear):
         return module(hidden_states)
-    return linear_epilogue(gemm_rows(hidden_states), module.dense.weight, module.dense.bias,
-                           None, GEMM_BIAS_GELU)
+    weight, bias = dense.weight, dense.bias
+    if not projection_on_hip(hidden_states, weight, bias):
+        return module(hidden_states)
+    return linear_epilogue(gemm_rows(hidden_states), weight, bias, None, GEMM_BIAS_GELU)
 
 
 def fusable_output_block(module: nn.Module) -> bool:
@@ -342,13 +362,13 @@ def output_block(module: nn.Module, hidden_states: torch.Tensor,
     """
 
     dense = module.dense
-    residual = input_tensor if input_tensor.is_contiguous() else input_tensor.contiguous()
+    residual = gemm_rows(input_tensor)
     norm = module.LayerNorm
-    if linear_fits(dense) and hidden_states.dtype == dense.weight.dtype \
-            and projection_on_hip(hidden_states, dense.out_features):
-        return linear_add_layernorm(gemm_rows(hidden_states), dense.weight, dense.bias, residual,
+    weight, bias = dense.weight, dense.bias
+    if isinstance(dense, nn.Linear) and projection_on_hip(hidden_states, weight, bias):
+        return linear_add_layernorm(gemm_rows(hidden_states), weight, bias, residual,
                                     norm.weight, norm.bias, norm.eps)
-    projected = F.linear(hidden_states, dense.weight, dense.bias)
+    projected = F.linear(hidden_states, weight, bias)
     return add_layernorm(projected, residual, norm.weight, norm.bias, norm.eps)
 
 

@@ -27,28 +27,20 @@ from .kernel import (
 MAX_ROWS = 4096
 
 
-def _linear_pointers(module: nn.Module, dtype: torch.dtype, device: torch.device, n: int,
-                     k: int) -> tuple[int, int] | None:
-    """Addresses of an ``[n, k]`` nn.Linear's weight and bias if the GEMM takes them."""
+def _pointers(module: nn.Module, dtype: torch.dtype, device: torch.device,
+              shape: tuple[int, ...]) -> tuple[int, int] | None:
+    """Addresses of the weight (of ``shape``) and bias of an nn.Linear or nn.LayerNorm if the
+    library takes them: one dtype, dense, 16-byte aligned."""
 
     parameters = module._parameters
     weight, bias = parameters.get("weight"), parameters.get("bias")
     if weight is None or bias is None or weight.dtype != dtype or bias.dtype != dtype \
-            or weight.shape != (n, k) or not weight.is_contiguous() or not bias.is_contiguous() \
+            or weight.shape != shape or bias.shape != shape[:1] \
+            or not weight.is_contiguous() or not bias.is_contiguous() \
             or weight.device != device or bias.device != device:
         return None
-    return weight.data_ptr(), bias.data_ptr()
-
-
-def _norm_pointers(module: nn.Module, dtype: torch.dtype,
-                   device: torch.device) -> tuple[int, int] | None:
-    parameters = module._parameters
-    weight, bias = parameters.get("weight"), parameters.get("bias")
-    if weight is None or bias is None or weight.dtype != dtype or bias.dtype != dtype \
-            or weight.device != device or bias.device != device \
-            or not weight.is_contiguous() or not bias.is_contiguous():
-        return None
-    return weight.data_ptr(), bias.data_ptr()
+    at = weight.data_ptr(), bias.data_ptr()
+    return at if (at[0] | at[1]) & 15 == 0 else None
 
 
 class NativeLayer:
@@ -75,19 +67,18 @@ class NativeLayer:
         inner_dense = self.intermediate._modules["dense"]
         inner = inner_dense.out_features
         if dim not in SUPPORTED_HEAD_DIMS or qkv.dtype != dtype or qkv.device != device \
-                or qkv.shape != (3 * width, hidden) \
-                or not layers.gemm_width_fits(3 * width, hidden) \
+                or qkv.shape != (3 * width, hidden) or not layers.gemm_fits(qkv, prep.qkv_bias) \
                 or not layers.gemm_width_fits(hidden, width) \
                 or not layers.gemm_width_fits(inner, hidden) \
                 or not layers.gemm_width_fits(hidden, inner):
             return None
         tail, last = self.attention_output._modules, self.output._modules
         attention_norm, output_norm = tail["LayerNorm"], last["LayerNorm"]
-        found = (_linear_pointers(tail["dense"], dtype, device, hidden, width),
-                 _norm_pointers(attention_norm, dtype, device),
-                 _linear_pointers(inner_dense, dtype, device, inner, hidden),
-                 _linear_pointers(last["dense"], dtype, device, hidden, inner),
-                 _norm_pointers(output_norm, dtype, device))
+        found = (_pointers(tail["dense"], dtype, device, (hidden, width)),
+                 _pointers(attention_norm, dtype, device, (hidden,)),
+                 _pointers(inner_dense, dtype, device, (inner, hidden)),
+                 _pointers(last["dense"], dtype, device, (hidden, inner)),
+                 _pointers(output_norm, dtype, device, (hidden,)))
         if None in found:
             return None
         has_c2p, has_p2c = attention.has_c2p, attention.has_p2c
@@ -103,8 +94,11 @@ class NativeLayer:
         if lut.dtype != torch.int32 or lut.device != device or lut.dim() != 1 \
                 or lut.numel() != 2 * x.shape[1] - 1 or not lut.is_contiguous():
             return None
+        qkv_at = qkv.data_ptr(), prep.qkv_bias.data_ptr()
+        if (qkv_at[0] | qkv_at[1]) & 15:
+            return None
         return _lib.EncoderLayer(
-            qkv.data_ptr(), prep.qkv_bias.data_ptr(),
+            *qkv_at,
             pos_key.data_ptr() if has_c2p else None, pos_query.data_ptr() if has_p2c else None,
             lut.data_ptr(), *found[0], *found[1], *found[2], *found[3], *found[4],
             attention.score_scale_log2(), attention_norm.eps, output_norm.eps,
@@ -124,13 +118,18 @@ class NativeForward:
     def covers(x: torch.Tensor, mask: torch.Tensor) -> bool:
         return (layers.USE_HIP_GEMM and layers.GEMM_CONFIG == 0 and x.dim() == 3
                 and x.dtype in layers.GEMM_DTYPES and 0 < x.shape[0] * x.shape[1] <= MAX_ROWS
-                and _lib.runs_directly(x) and x.is_contiguous()
+                and _lib.runs_directly(x)
                 and type(mask) is torch.Tensor and mask.device == x.device
                 and mask.shape == x.shape[:2] and mask.dtype == torch.bool
                 and mask.is_contiguous())
 
     def run(self, layer: NativeLayer, x: torch.Tensor,
             plan: HipPreparedPositionPlan) -> torch.Tensor | None:
+        # A layer's input may come from a step run op by op (the first layer's from the
+        # caller, the second's from the convolution), so each is looked at.
+        if x.shape[:2] != self.mask.shape or not _lib.runs_directly(x) \
+                or not x.is_contiguous() or x.data_ptr() & 15:
+            return None
         layer.attention._validate_hip_call(x)
         batch, length = x.shape[:2]
         if length != plan.sequence_length:
