@@ -14,12 +14,15 @@ from __future__ import annotations
 import ctypes
 import functools
 import os
+import struct
 from pathlib import Path
 
 import torch  # noqa: F401  (load torch's HIP runtime first)
 
 LIBRARY_NAME = "libdflash.so"
 ABI_VERSION = 7
+
+ERR_WORKSPACE = -7  # DFLASH_ERR_WORKSPACE
 
 DTYPE_CODES = {
     torch.float16: 0,
@@ -44,6 +47,9 @@ class EncoderLayer(ctypes.Structure):
         (name, _c_float) for name in ("score_scale_log2", "attention_eps", "output_eps")] + [
         (name, _c_int) for name in ("heads", "head_dim", "slots", "hidden", "inner", "dtype")]
 
+
+# The same fields for struct.pack (a Structure takes its fields one by one, 3 us).
+ENCODER_LAYER_FORMAT = struct.Struct("@15P3f6i0P")
 
 _handle: ctypes.CDLL | None = None
 _load_error: str | None = None
@@ -179,7 +185,7 @@ def check(code: int, what: str) -> None:
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
-_PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
+PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 try:
     from torch.utils._python_dispatch import _get_current_dispatch_mode as _get_dispatch_mode
@@ -200,7 +206,7 @@ def runs_directly(tensor: torch.Tensor) -> bool:
     """True outside tracing (torch.compile, export) and dispatch modes, for a plain CUDA
     tensor: the library may be called on its address."""
 
-    return (type(tensor) in _PLAIN_TENSORS and tensor.device.type == "cuda"
+    return (type(tensor) in PLAIN_TENSORS and tensor.device.type == "cuda"
             and not torch.compiler.is_compiling() and _get_dispatch_mode() is None)
 
 
@@ -228,7 +234,7 @@ def hip_op(name: str):
                 return op(*args, **kwargs)
             for a in args:
                 if isinstance(a, torch.Tensor) and (
-                        type(a) not in _PLAIN_TENSORS or a.device.type != "cuda"):
+                        type(a) not in PLAIN_TENSORS or a.device.type != "cuda"):
                     return op(*args, **kwargs)
             return impl(*args, **kwargs)
 

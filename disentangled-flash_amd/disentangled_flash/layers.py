@@ -26,6 +26,7 @@ import threading
 import torch
 from torch import nn
 from torch.nn import functional as F
+from torch.nn.modules import module as torch_module
 
 from . import _lib
 
@@ -300,9 +301,11 @@ def fusable_intermediate(module: nn.Module) -> bool:
     or ``torch.nn.functional.gelu`` itself.
     """
 
-    if not linear_fits(getattr(module, "dense", None)):
-        return False
-    act = getattr(module, "intermediate_act_fn", None)
+    return linear_fits(getattr(module, "dense", None)) \
+        and _is_erf_gelu(getattr(module, "intermediate_act_fn", None))
+
+
+def _is_erf_gelu(act) -> bool:
     if act is F.gelu:
         return True
     if type(act).__name__ != "GELUActivation":
@@ -311,13 +314,35 @@ def fusable_intermediate(module: nn.Module) -> bool:
     return inner is F.gelu or getattr(inner, "__name__", "") == "_gelu_python"
 
 
+def _is_plain_call(module: nn.Module) -> bool:
+    """True if ``module(x)`` is its class's ``forward`` and nothing else: no forward hooks of
+    its own, no ``forward`` set on the instance."""
+
+    return not (module._forward_hooks or module._forward_pre_hooks
+                or "forward" in module.__dict__)
+
+
+def intermediate_is_dense_gelu(module: nn.Module) -> bool:
+    """True if calling ``module`` (a :func:`fusable_intermediate` when the encoder was prepared)
+    still is its dense layer and an erf GELU: nothing was hooked, wrapped or replaced."""
+
+    modules = module._modules  # (past nn.Module's attribute lookup: this runs on every call)
+    dense, act = modules.get("dense"), modules.get("intermediate_act_fn")
+    if act is None:
+        act = module.__dict__.get("intermediate_act_fn")
+    return isinstance(dense, nn.Linear) and _is_plain_call(module) and _is_plain_call(dense) \
+        and _is_erf_gelu(act) and (act is F.gelu or _is_plain_call(act)) \
+        and not (torch_module._global_forward_hooks or torch_module._global_forward_pre_hooks)
+
+
 def intermediate_block(module: nn.Module, hidden_states: torch.Tensor) -> torch.Tensor:
     """``module(hidden_states)`` as one GEMM with the GELU in its epilogue, or the
-    module itself where :func:`projection_on_hip` says so."""
+    module itself where it has hooks or another activation, or where
+    :func:`projection_on_hip` says so."""
 
-    dense = module.dense
-    if not isinstance(dense, nn.Linear):
+    if not torch.compiler.is_compiling() and not intermediate_is_dense_gelu(module):
         return module(hidden_states)
+    dense = module.dense
     weight, bias = dense.weight, dense.bias
     if not projection_on_hip(hidden_states, weight, bias):
         return module(hidden_states)

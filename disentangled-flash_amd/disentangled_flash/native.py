@@ -27,20 +27,30 @@ from .kernel import (
 MAX_ROWS = 4096
 
 
-def _pointers(module: nn.Module, dtype: torch.dtype, device: torch.device,
-              shape: tuple[int, ...]) -> tuple[int, int] | None:
-    """Addresses of the weight (of ``shape``) and bias of an nn.Linear or nn.LayerNorm if the
-    library takes them: one dtype, dense, 16-byte aligned."""
+_Attention = HipInferenceDisentangledSelfAttention
+_FORWARD_PREPARED = _Attention.forward_prepared
+_FUSED_PROJECTION = _Attention._fused_projection
 
-    parameters = module._parameters
-    weight, bias = parameters.get("weight"), parameters.get("bias")
-    if weight is None or bias is None or weight.dtype != dtype or bias.dtype != dtype \
-            or weight.shape != shape or bias.shape != shape[:1] \
-            or not weight.is_contiguous() or not bias.is_contiguous() \
-            or weight.device != device or bias.device != device:
-        return None
-    at = weight.data_ptr(), bias.data_ptr()
-    return at if (at[0] | at[1]) & 15 == 0 else None
+
+def _runs_as_written(attention: nn.Module) -> bool:
+    """False where a subclass or the instance overrides what the library call stands for."""
+
+    state = attention.__dict__
+    return type(attention) is _Attention and _Attention.forward_prepared is _FORWARD_PREPARED \
+        and _Attention._fused_projection is _FUSED_PROJECTION \
+        and "forward_prepared" not in state and "_fused_projection" not in state
+
+
+def _taken(weight: torch.Tensor | None, bias: torch.Tensor | None, dtype: torch.dtype,
+           device: int, shape: tuple[int, ...]) -> bool:
+    """True if the library takes a weight of ``shape`` and its bias: one dtype, one device,
+    dense."""
+
+    return (weight is not None and bias is not None
+            and weight.dtype is dtype and bias.dtype is dtype
+            and weight.shape == shape and bias.shape == shape[:1]
+            and weight.get_device() == device and bias.get_device() == device
+            and weight.is_contiguous() and bias.is_contiguous())
 
 
 class NativeLayer:
@@ -58,51 +68,67 @@ class NativeLayer:
 
         attention = self.attention
         prep = attention._prepared
-        if prep is None or prep.qkv_bias is None or attention.relative_mode != "fused":
+        if prep is None or attention.relative_mode != "fused" or not _runs_as_written(attention) \
+                or not layers.intermediate_is_dense_gelu(self.intermediate):
             return None
-        dtype, device, hidden = x.dtype, x.device, x.shape[-1]
+        dtype, device, (_, length, hidden) = x.dtype, x.get_device(), x.shape
         heads, dim = attention.num_attention_heads, attention.attention_head_size
         width = heads * dim
-        qkv = prep.qkv_weight
         inner_dense = self.intermediate._modules["dense"]
         inner = inner_dense.out_features
-        if dim not in SUPPORTED_HEAD_DIMS or qkv.dtype != dtype or qkv.device != device \
-                or qkv.shape != (3 * width, hidden) or not layers.gemm_fits(qkv, prep.qkv_bias) \
+        if dim not in SUPPORTED_HEAD_DIMS or dtype not in layers.GEMM_DTYPES \
+                or not layers.gemm_width_fits(3 * width, hidden) \
                 or not layers.gemm_width_fits(hidden, width) \
                 or not layers.gemm_width_fits(inner, hidden) \
                 or not layers.gemm_width_fits(hidden, inner):
             return None
         tail, last = self.attention_output._modules, self.output._modules
         attention_norm, output_norm = tail["LayerNorm"], last["LayerNorm"]
-        found = (_pointers(tail["dense"], dtype, device, (hidden, width)),
-                 _pointers(attention_norm, dtype, device, (hidden,)),
-                 _pointers(inner_dense, dtype, device, (inner, hidden)),
-                 _pointers(last["dense"], dtype, device, (hidden, inner)),
-                 _pointers(output_norm, dtype, device, (hidden,)))
-        if None in found:
+        addresses = []
+        for parameters, shape in ((tail["dense"]._parameters, (hidden, width)),
+                                  (attention_norm._parameters, (hidden,)),
+                                  (inner_dense._parameters, (inner, hidden)),
+                                  (last["dense"]._parameters, (hidden, inner)),
+                                  (output_norm._parameters, (hidden,))):
+            weight, bias = parameters.get("weight"), parameters.get("bias")
+            if not _taken(weight, bias, dtype, device, shape):
+                return None
+            addresses += weight.data_ptr(), bias.data_ptr()
+        qkv, qkv_bias = prep.qkv_weight, prep.qkv_bias
+        if not _taken(qkv, qkv_bias, dtype, device, (3 * width, hidden)):
             return None
-        has_c2p, has_p2c = attention.has_c2p, attention.has_p2c
-        pos_key, pos_query = plan.pos_key, plan.pos_query
-        slots = 0
-        for rows in ((pos_key,) if has_c2p else ()) + ((pos_query,) if has_p2c else ()):
-            if rows is None or rows.dtype != dtype or rows.device != device \
-                    or rows.dim() != 3 or rows.size(0) != heads or rows.size(2) != dim \
-                    or not rows.is_contiguous() or (slots and rows.size(1) != slots):
+        qkv, qkv_bias = qkv.data_ptr(), qkv_bias.data_ptr()
+        pos_key = pos_query = slots = 0
+        rows = plan.pos_key
+        if attention.has_c2p:
+            if rows is None or rows.dtype is not dtype or rows.get_device() != device \
+                    or rows.dim() != 3 or not rows.is_contiguous():
+                return None
+            at, slots, row = rows.shape
+            if at != heads or row != dim:
+                return None
+            pos_key = rows.data_ptr()
+        rows = plan.pos_query
+        if attention.has_p2c:
+            if rows is None or rows.dtype is not dtype or rows.get_device() != device \
+                    or rows.dim() != 3 or not rows.is_contiguous() \
+                    or rows.shape != (heads, slots or rows.size(1), dim):
                 return None
             slots = rows.size(1)
+            pos_query = rows.data_ptr()
         lut = plan.delta_to_local
-        if lut.dtype != torch.int32 or lut.device != device or lut.dim() != 1 \
-                or lut.numel() != 2 * x.shape[1] - 1 or not lut.is_contiguous():
+        if lut.dtype is not torch.int32 or lut.get_device() != device \
+                or lut.shape != (2 * length - 1,) or not lut.is_contiguous():
             return None
-        qkv_at = qkv.data_ptr(), prep.qkv_bias.data_ptr()
-        if (qkv_at[0] | qkv_at[1]) & 15:
+        misaligned = qkv | qkv_bias
+        for at in addresses:
+            misaligned |= at
+        if misaligned & 15:
             return None
-        return _lib.EncoderLayer(
-            *qkv_at,
-            pos_key.data_ptr() if has_c2p else None, pos_query.data_ptr() if has_p2c else None,
-            lut.data_ptr(), *found[0], *found[1], *found[2], *found[3], *found[4],
+        return _lib.EncoderLayer.from_buffer_copy(_lib.ENCODER_LAYER_FORMAT.pack(
+            qkv, qkv_bias, pos_key, pos_query, lut.data_ptr(), *addresses,
             attention.score_scale_log2(), attention_norm.eps, output_norm.eps,
-            heads, dim, slots, hidden, inner, _lib.DTYPE_CODES[dtype])
+            heads, dim, slots, hidden, inner, _lib.DTYPE_CODES[dtype]))
 
 
 class NativeForward:
@@ -111,6 +137,8 @@ class NativeForward:
     def __init__(self, x: torch.Tensor, mask: torch.Tensor) -> None:
         self.lib = _lib.load()
         self.mask = mask
+        self.shape = tuple(mask.shape)
+        self.device = x.get_device()
         self.workspace: torch.Tensor | None = None
         self.stream = _lib.current_stream_handle(x.device)
 
@@ -126,29 +154,38 @@ class NativeForward:
     def run(self, layer: NativeLayer, x: torch.Tensor,
             plan: HipPreparedPositionPlan) -> torch.Tensor | None:
         # A layer's input may come from a step run op by op (the first layer's from the
-        # caller, the second's from the convolution), so each is looked at.
-        if x.shape[:2] != self.mask.shape or not _lib.runs_directly(x) \
-                or not x.is_contiguous() or x.data_ptr() & 15:
+        # caller, the second's from the convolution), so each is looked at; what only the
+        # op-by-op path reports (training, gradients, another length) is left to it.
+        if type(x) not in _lib.PLAIN_TENSORS or x.dim() != 3 or not x.is_contiguous() \
+                or x.data_ptr() & 15 or x.get_device() != self.device:
             return None
-        layer.attention._validate_hip_call(x)
-        batch, length = x.shape[:2]
-        if length != plan.sequence_length:
-            return None  # the op-by-op path reports it
+        batch, length, _ = x.shape
+        if (batch, length) != self.shape or length != plan.sequence_length \
+                or layer.attention.training or torch.is_grad_enabled():
+            return None
         described = layer.describe(x, plan)
         if described is None:
             return None
         reference = ctypes.byref(described)
-        size = self.lib.dflash_encoder_layer_workspace_bytes(reference, batch, length)
-        if size == 0:
-            return None
-        if self.workspace is None or self.workspace.numel() < size:
-            self.workspace = torch.empty(size, device=x.device, dtype=torch.uint8)
         out = torch.empty_like(x)
-        code = self.lib.dflash_encoder_layer_fwd(
-            reference, x.data_ptr(), self.mask.data_ptr(), out.data_ptr(), batch, length,
-            self.workspace.data_ptr(), self.workspace.numel(), self.stream)
+        # The layers of a forward are mostly alike: the library says when one needs more
+        # workspace (before it launches anything).
+        code = _lib.ERR_WORKSPACE
+        if self.workspace is not None:
+            code = self.run_layer(reference, x, out)
+        if code == _lib.ERR_WORKSPACE:
+            size = self.lib.dflash_encoder_layer_workspace_bytes(reference, batch, length)
+            if size == 0:
+                return None
+            self.workspace = torch.empty(size, device=x.device, dtype=torch.uint8)
+            code = self.run_layer(reference, x, out)
         _lib.check(code, "dflash_encoder_layer_fwd")
         return out
+
+    def run_layer(self, reference, x: torch.Tensor, out: torch.Tensor) -> int:
+        return self.lib.dflash_encoder_layer_fwd(
+            reference, x.data_ptr(), self.mask.data_ptr(), out.data_ptr(), *self.shape,
+            self.workspace.data_ptr(), self.workspace.numel(), self.stream)
 
 
 __all__ = ["MAX_ROWS", "NativeForward", "NativeLayer"]
