@@ -105,7 +105,7 @@ int dflash_attention_fwd(const void* query, const void* key, const void* value, 
   // reference's TF32 mode, kernel.py:222); the windows are read, not multiplied.
   rp.fast = (dtype == DFLASH_DTYPE_FP32 && !strict_fp32) ? 1 : 0;
   rp.table = 1;
-  return launch_rel_attention(rp, D, dtype, static_cast<hipStream_t>(stream));
+  return launch_rel_attention(rp, D, dtype, 0, static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"
@@ -188,8 +188,8 @@ int rel_forward(const void* query, const void* key, const void* value, int64_t s
   rp.has_c2p = has_c2p;
   rp.has_p2c = has_p2c;
   rp.splits = 1;
-  rp.cus = current_device_cus();
-  rp.qw = rel_attention_qw(B, H, L, D, rp.cus, has_c2p != 0);
+  const int cus = current_device_cus();
+  rp.qw = rel_attention_qw(B, H, L, D, cus, has_c2p != 0);
   rp.fast = dtype == DFLASH_DTYPE_FP32 && !strict_fp32;
   if (splits > 1 && dtype != DFLASH_DTYPE_FP32) {  // fp32 runs unsplit
     if (splits > 8) return DFLASH_ERR_SHAPE;
@@ -206,7 +206,7 @@ int rel_forward(const void* query, const void* key, const void* value, int64_t s
       rp.part = static_cast<float*>(workspace);
     }
   }
-  return launch_rel_attention(rp, D, dtype, static_cast<hipStream_t>(stream));
+  return launch_rel_attention(rp, D, dtype, cus, static_cast<hipStream_t>(stream));
 }
 
 constexpr int kMaxDevices = 64;

@@ -41,14 +41,13 @@ struct RelParams {
   // last slice, b = B - 1 and h = H - 1, may run as a launch of its own); 0
   // otherwise.
   int bh0;
-  int cus;        // CUs of the device
-  int by_length;  // 1 = the longest sequences of the batch first, set by the launcher
 };
 
 // fp16 / bf16 / fp32, D in {32, 64, 128}; arguments already validated by the
 // caller.  prm.splits / split_tiles / part select the split-key form (with its
 // merge; 16-bit types only).
-int launch_rel_attention(const RelParams& prm, int D, int dtype, hipStream_t stream);
+// (cus: the device's CUs, which the order of the sequences depends on.)
+int launch_rel_attention(const RelParams& prm, int D, int dtype, int cus, hipStream_t stream);
 
 // Key splits for a launch of B*H query-block rows that would leave the GPU
 // underfilled (fewer workgroups than two per CU), and the workspace bytes they

@@ -393,14 +393,15 @@ struct RelLayout {
 // the end of L), one byte per lane and one load in all: with eight probes a lane the
 // order cost 1.2 us a workgroup.  A mask with holes only makes the order worse; it is
 // a permutation for any mask.
-// Probe and order are two steps so that loads of other things go out in between.
+// Probe and order are two steps so that the lookups go out in between.
 constexpr int kSortBatch = 16;
-// Built for the forms of one workgroup per CU (fp32, and 16-bit d = 128 on the 32-row
-// tile), whose workgroups are the long ones.  With two per CU a CU evens them out by
-// itself: d = 64 ragged 52.2 -> 51.5 us but full 87.4 -> 88.9, d = 32 full 27.8 -> 28.7.
-template <int WGS, bool SPLIT, bool TABLE>
+// Built, as instances of their own, for the forms of one workgroup per CU (fp32, and
+// 16-bit d = 128 on the 32-row tile), whose workgroups are the long ones.  With two per CU
+// a CU evens them out by itself: d = 64 ragged 52.2 -> 51.5 us but full 87.4 -> 88.9,
+// d = 32 full 27.8 -> 28.7.
+template <int WGS, bool TABLE>
 constexpr bool rel_by_length() {
-  return WGS == 1 && !SPLIT && !TABLE;
+  return WGS == 1 && !TABLE;
 }
 __device__ inline uint8_t length_probe(const uint8_t* mask, int B, int L, int place) {
   const int lane = threadIdx.x & 63;
@@ -414,24 +415,31 @@ __device__ inline int sequence_by_length(uint8_t probe, int B, int place) {
   const int first = place & ~(kSortBatch - 1);
   const int count = min(B - first, kSortBatch);
   const uint64_t kept = __ballot(probe != 0);
-  const bool valid = lane < count;
-  const int n = valid ? __popc(static_cast<uint32_t>(kept >> (4 * lane & 63)) & 15u) : -1;
-  int before = 0;  // sequences longer than the present length
-  int at = -1;     // place of this lane's sequence
+  const int n = lane < count ? __popc(static_cast<uint32_t>(kept >> (4 * lane & 63)) & 15u) : -1;
+  // The sequences of the length that holds the place, and the place among them.
+  uint32_t pick = 0;
+  int at = place - first;
 #pragma unroll
   for (int v = 4; v >= 0; --v) {
     const uint32_t same = static_cast<uint32_t>(__ballot(n == v));
-    const int rank = __builtin_amdgcn_mbcnt_lo(same, static_cast<uint32_t>(before));
-    if (n == v) at = rank;
-    before += __popc(same);
+    const int many = __popc(same);
+    if (pick == 0) {
+      if (at < many) {
+        pick = same;
+      } else {
+        at -= many;
+      }
+    }
   }
-  return first + __builtin_ctz(static_cast<uint32_t>(__ballot(valid && at == place - first)));
+  const bool here = (pick >> (lane & 31) & 1u) != 0 && lane < 32 &&
+                    static_cast<int>(__builtin_amdgcn_mbcnt_lo(pick, 0u)) == at;
+  return first + __builtin_ctz(static_cast<uint32_t>(__ballot(here)));
 }
 
 }  // namespace
 
 template <typename T, int D, int QW, int BN, int VBUFS, int WGS, bool C2P, bool P2C, bool SPLIT,
-          bool FAST = false, bool TABLE = false, bool ROWSAFE = false>
+          bool FAST = false, bool TABLE = false, bool ROWSAFE = false, bool BY_LENGTH = false>
 __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams p) {
   static_assert(!FAST || sizeof(T) == 4, "the bf16x3 form is for fp32 data");
   static_assert(!(TABLE && SPLIT), "the table form runs unsplit");
@@ -495,14 +503,12 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
   const int g = lane >> 4;
 
   const int L = p.L;
-  int split = 0, qblk, b, h;
-  constexpr bool kByLength = rel_by_length<WGS, SPLIT, TABLE>();
-  bool by_length = false;
+  int split, qblk, b, h;
   uint8_t length = 0;
-  if constexpr (kByLength) by_length = p.by_length != 0;
-  if (by_length) {
+  if constexpr (BY_LENGTH) {
     // Groups dealt to the XCDs in turn (the last groups % 8 split by block), the
     // longest sequences of the batch first.
+    split = 0;
     const int groups = p.B * p.H;
     const int per = groups / 8;
     const int n = blockIdx.x;
@@ -516,10 +522,9 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
       group = 8 * per + l / p.nqb;
       qblk = l % p.nqb;
     }
-    const int place = group / p.H;  // of the sequence, by length
-    h = group - place * p.H;
-    b = place;
-    length = length_probe(p.mask, p.B, L, place);
+    b = group / p.H;  // the place of the sequence by length, until the order is known
+    h = group - b * p.H;
+    length = length_probe(p.mask, p.B, L, b);
   } else {
     const int mk = xcd_logical_block(blockIdx.x, gridDim.x);
     // Key split of the split-key form (the splits of a block are neighbours).
@@ -541,16 +546,12 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
   const uint32_t sl_bytes = static_cast<uint32_t>(p.sl) * ES;
 
   // Buffer resources.  Rows past L read as zero; the bound is the end of row L-1.
-  __amdgpu_buffer_rsrc_t rq, rk, rv, rmask;
-  auto set_sequence = [&]() {
-    const uint32_t head_bytes = (static_cast<uint32_t>(L - 1) * static_cast<uint32_t>(p.sl) + D) * ES;
-    const int64_t head_off = static_cast<int64_t>(b) * p.sb + static_cast<int64_t>(h) * p.sh;
-    rq = make_rsrc(reinterpret_cast<const T*>(p.q) + head_off, head_bytes);
-    rk = make_rsrc(reinterpret_cast<const T*>(p.k) + head_off, head_bytes);
-    rv = make_rsrc(reinterpret_cast<const T*>(p.v) + head_off, head_bytes);
-    rmask = make_rsrc(p.mask + static_cast<int64_t>(b) * L, static_cast<uint32_t>(L));
-  };
-  if constexpr (!kByLength) set_sequence();
+  const uint32_t head_bytes = (static_cast<uint32_t>(L - 1) * static_cast<uint32_t>(p.sl) + D) * ES;
+  const int64_t head_off = static_cast<int64_t>(b) * p.sb + static_cast<int64_t>(h) * p.sh;
+  auto rq = make_rsrc(reinterpret_cast<const T*>(p.q) + head_off, head_bytes);
+  auto rk = make_rsrc(reinterpret_cast<const T*>(p.k) + head_off, head_bytes);
+  auto rv = make_rsrc(reinterpret_cast<const T*>(p.v) + head_off, head_bytes);
+  auto rmask = make_rsrc(p.mask + static_cast<int64_t>(b) * L, static_cast<uint32_t>(L));
   const uint32_t rel_bytes = static_cast<uint32_t>(p.S) * D * ES;
   const auto rkr = make_rsrc(reinterpret_cast<const T*>(p.pos_key) + static_cast<int64_t>(h) * p.S * D,
                              rel_bytes);
@@ -1061,9 +1062,13 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
     for (int u = 0; u < PU; ++u) lp[u] = lut_load(lut_p_index(jstart, u));
     lutp = lut_load(lut_p_index(jstart + BN, 0));
   }
-  if constexpr (kByLength) {
-    if (by_length) b = sequence_by_length(length, p.B, b);
-    set_sequence();
+  if constexpr (BY_LENGTH) {
+    b = sequence_by_length(length, p.B, b);
+    const int64_t off = static_cast<int64_t>(b) * p.sb + static_cast<int64_t>(h) * p.sh;
+    rq = make_rsrc(reinterpret_cast<const T*>(p.q) + off, head_bytes);
+    rk = make_rsrc(reinterpret_cast<const T*>(p.k) + off, head_bytes);
+    rv = make_rsrc(reinterpret_cast<const T*>(p.v) + off, head_bytes);
+    rmask = make_rsrc(p.mask + static_cast<int64_t>(b) * L, static_cast<uint32_t>(L));
   }
   // Mask bytes: the first 512 of the sequence (for the extent), the
   // workgroup's queries and each lane's queries.  Bytes past L read as zero.
@@ -1082,31 +1087,29 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
   // Workgroup and query flags from the mask bytes.
   bool wg_kept = false;
   bool wg_padded = false;
-  if constexpr (!kByLength) {
 #pragma unroll
-    for (int n = 0; n < kWgMaskLoads; ++n) {
-      const bool mine = 64 * n + lane < BM;
-      const bool kept = wm[n] != 0;
-      wg_kept = wg_kept || __any(kept);
-      wg_padded = wg_padded || __any(mine && i0 + 64 * n + lane < L && !kept);
-    }
+  for (int n = 0; n < kWgMaskLoads; ++n) {
+    const bool mine = 64 * n + lane < BM;
+    const bool kept = wm[n] != 0;
+    wg_kept = wg_kept || __any(kept);
+    wg_padded = wg_padded || __any(mine && i0 + 64 * n + lane < L && !kept);
+  }
 #pragma unroll
-    for (int qb = 0; qb < kQB; ++qb) qkept[qb] = qm[qb] != 0;
+  for (int qb = 0; qb < kQB; ++qb) qkept[qb] = qm[qb] != 0;
 
-    if (!wg_kept) {
-      if (SPLIT && split > 0) return;  // split 0 stores the mean of V
-      // Every query of the workgroup is padded (or past L): all rows are the mean of V.
-      v_mean();
-      const int row_lo = i0 + tid / (D / 4);
-      for (int i = row_lo; i < min(i0 + BM, L); i += kThreads / (D / 4)) {
-        const int d0 = 4 * (tid % (D / 4));
-        Quad<T> q;
+  if (!wg_kept) {
+    if (SPLIT && split > 0) return;  // split 0 stores the mean of V
+    // Every query of the workgroup is padded (or past L): all rows are the mean of V.
+    v_mean();
+    const int row_lo = i0 + tid / (D / 4);
+    for (int i = row_lo; i < min(i0 + BM, L); i += kThreads / (D / 4)) {
+      const int d0 = 4 * (tid % (D / 4));
+      Quad<T> q;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) q[r] = static_cast<T>(vmean[d0 + r]);
-        *reinterpret_cast<Quad<T>*>(outp + (static_cast<int64_t>(b) * L + i) * row_stride + h * D + d0) = q;
-      }
-      return;
+      for (int r = 0; r < 4; ++r) q[r] = static_cast<T>(vmean[d0 + r]);
+      *reinterpret_cast<Quad<T>*>(outp + (static_cast<int64_t>(b) * L + i) * row_stride + h * D + d0) = q;
     }
+    return;
   }
 
   // Rows of the tile-0 windows, then Q and the K/V of tile 0 (a workgroup
@@ -1148,34 +1151,6 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
   } else {
     prefetch_k(jstart);
     prefetch_v(jstart);
-  }
-  // By length, the mask bytes came a load later than the lookups, and the loads above
-  // went out without waiting for them (d = 128 ragged 66.1 against 66.7 us waiting).
-  if constexpr (kByLength) {
-#pragma unroll
-    for (int n = 0; n < kWgMaskLoads; ++n) {
-      const bool mine = 64 * n + lane < BM;
-      const bool kept = wm[n] != 0;
-      wg_kept = wg_kept || __any(kept);
-      wg_padded = wg_padded || __any(mine && i0 + 64 * n + lane < L && !kept);
-    }
-#pragma unroll
-    for (int qb = 0; qb < kQB; ++qb) qkept[qb] = qm[qb] != 0;
-
-    if (!wg_kept) {
-      if constexpr (kDirect) wait_vmem<0>();  // the copies land before LDS is reused
-      // Every query of the workgroup is padded (or past L): all rows are the mean of V.
-      v_mean();
-      const int row_lo = i0 + tid / (D / 4);
-      for (int i = row_lo; i < min(i0 + BM, L); i += kThreads / (D / 4)) {
-        const int d0 = 4 * (tid % (D / 4));
-        Quad<T> q;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) q[r] = static_cast<T>(vmean[d0 + r]);
-        *reinterpret_cast<Quad<T>*>(outp + (static_cast<int64_t>(b) * L + i) * row_stride + h * D + d0) = q;
-      }
-      return;
-    }
   }
   // Tile 1 (d = 64 only: d = 128 has no registers to spare here, and d = 32,
   // whose tiles are short, measured faster without it): K/V and the rows of
@@ -1908,7 +1883,7 @@ __global__ __launch_bounds__(256) void rel_split_merge_kernel(const float* __res
 }
 
 template <typename T, int D, int QW, bool C2P, bool P2C, bool FAST = false, bool TABLE = false>
-int launch_rel(const RelParams& base, hipStream_t stream) {
+int launch_rel(const RelParams& base, int cus, hipStream_t stream) {
   constexpr int BN = rel_block_n<D>();
   constexpr int VB = rel_v_buffers<T, D, QW, FAST, C2P>();
   constexpr int WGS = rel_workgroups_per_cu<T, D, QW>();
@@ -1917,12 +1892,14 @@ int launch_rel(const RelParams& base, hipStream_t stream) {
   RelParams prm = base;
   prm.nqb = (prm.L + LY::BM - 1) / LY::BM;
   // Longest sequences first where the grid runs in more than one round: the last round
-  // then holds the short ones (fp32 d = 64, H = 12, L = 384, B = 8 ragged 91.1 -> 77.5
-  // us; B = 30, L = 300, H = 6 95.2 -> 89.4; d = 128, H = 8, L = 512, B = 16 ragged 71.3
-  // -> 66.1).  With every sequence full it buys nothing and costs under 1 us a launch
-  // (fp32 107.0 -> 108.6, d = 128 72.1 -> 72.4).  A single round starts all at once.
-  prm.by_length = rel_by_length<WGS, false, TABLE>() && prm.B > 1 && prm.splits <= 1 &&
-                  static_cast<int64_t>(prm.nqb) * prm.B * prm.H > prm.cus;
+  // then holds the short ones (ragged, fp32 d = 64, H = 12, L = 384, B = 8 92.0 -> 77.9 us;
+  // B = 30, L = 300, H = 6 96.1 -> 89.9; fp32 d = 32 90.8 -> 86.0, d = 128 201.6 -> 184.2;
+  // fp16 d = 128, H = 8, L = 512, B = 16 72.0 -> 65.0).  With every sequence full it buys
+  // nothing and costs the order (fp32 d = 64 108.2 -> 108.4, d = 32, three rounds, 95.4 ->
+  // 96.5, d = 128 213.5 -> 214.9; fp16 d = 128 72.8 -> 72.1).  A single round starts all at
+  // once.
+  const bool by_length = rel_by_length<WGS, TABLE>() && prm.B > 1 && prm.splits <= 1 &&
+                         static_cast<int64_t>(prm.nqb) * prm.B * prm.H > cus;
   // The split-key form exists for the default 16-bit tile (QW = 32 at d <= 64,
   // 16 at d = 128); fp32 never splits.
   constexpr bool kSplitBuilt = sizeof(T) == 2 && (D >= 128 ? QW == 16 : QW == 32) && !TABLE;
@@ -1941,7 +1918,17 @@ int launch_rel(const RelParams& base, hipStream_t stream) {
                          LY::bytes, stream, prm);
     }
   }
-  if (prm.splits <= 1) {
+  if constexpr (rel_by_length<WGS, TABLE>()) {
+    constexpr auto ordered_kernel =
+        rel_attention_kernel<T, D, QW, BN, VB, WGS, C2P, P2C, false, FAST, TABLE, false, true>;
+    if (by_length) {
+      err = ensure_dynamic_lds<ordered_kernel>(static_cast<int>(LY::bytes));
+      if (err != hipSuccess) return static_cast<int>(err);
+      hipLaunchKernelGGL(ordered_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads),
+                         LY::bytes, stream, prm);
+    }
+  }
+  if (prm.splits <= 1 && !by_length) {
     err = ensure_dynamic_lds<kernel>(static_cast<int>(LY::bytes));
     if (err != hipSuccess) return static_cast<int>(err);
     // Table form with L not a multiple of the tiles: the last (b, h) slice,
@@ -1978,23 +1965,23 @@ int launch_rel(const RelParams& base, hipStream_t stream) {
 }
 
 template <typename T, int D, int QW, bool FAST = false>
-int rel_modes_qw(const RelParams& prm, hipStream_t stream) {
+int rel_modes_qw(const RelParams& prm, int cus, hipStream_t stream) {
   if constexpr (sizeof(T) == 4 && !FAST) {
-    if (prm.fast) return rel_modes_qw<T, D, QW, true>(prm, stream);
+    if (prm.fast) return rel_modes_qw<T, D, QW, true>(prm, cus, stream);
   }
   // Table form: the default tile of each head dim, 16-bit or fp32 (IEEE, or
   // the bf16x3 products of the fast form for QK and PV).
   if constexpr (QW == (D >= 128 ? 16 : 32)) {
     if (prm.table) {
-      if (prm.has_c2p && prm.has_p2c) return launch_rel<T, D, QW, true, true, FAST, true>(prm, stream);
-      if (prm.has_c2p) return launch_rel<T, D, QW, true, false, FAST, true>(prm, stream);
-      if (prm.has_p2c) return launch_rel<T, D, QW, false, true, FAST, true>(prm, stream);
+      if (prm.has_c2p && prm.has_p2c) return launch_rel<T, D, QW, true, true, FAST, true>(prm, cus, stream);
+      if (prm.has_c2p) return launch_rel<T, D, QW, true, false, FAST, true>(prm, cus, stream);
+      if (prm.has_p2c) return launch_rel<T, D, QW, false, true, FAST, true>(prm, cus, stream);
     }
   }
-  if (prm.has_c2p && prm.has_p2c) return launch_rel<T, D, QW, true, true, FAST>(prm, stream);
-  if (prm.has_c2p) return launch_rel<T, D, QW, true, false, FAST>(prm, stream);
-  if (prm.has_p2c) return launch_rel<T, D, QW, false, true, FAST>(prm, stream);
-  return launch_rel<T, D, QW, false, false, FAST>(prm, stream);
+  if (prm.has_c2p && prm.has_p2c) return launch_rel<T, D, QW, true, true, FAST>(prm, cus, stream);
+  if (prm.has_c2p) return launch_rel<T, D, QW, true, false, FAST>(prm, cus, stream);
+  if (prm.has_p2c) return launch_rel<T, D, QW, false, true, FAST>(prm, cus, stream);
+  return launch_rel<T, D, QW, false, false, FAST>(prm, cus, stream);
 }
 
 // 16-bit d = 128 runs QW = 32 (one workgroup per CU, 512 registers per lane)
@@ -2004,17 +1991,17 @@ int rel_modes_qw(const RelParams& prm, hipStream_t stream) {
 // only QW = 32 (QW = 16 measured 1.2-2.5x slower at every batch, see
 // rel_attention_qw).
 template <typename T, int D>
-int rel_modes(const RelParams& prm, hipStream_t stream) {
+int rel_modes(const RelParams& prm, int cus, hipStream_t stream) {
   if constexpr (D >= 128 && sizeof(T) == 2) {
-    if (prm.qw == 32 && prm.splits <= 1) return rel_modes_qw<T, D, 32>(prm, stream);
-    return rel_modes_qw<T, D, 16>(prm, stream);
+    if (prm.qw == 32 && prm.splits <= 1) return rel_modes_qw<T, D, 32>(prm, cus, stream);
+    return rel_modes_qw<T, D, 16>(prm, cus, stream);
   } else if constexpr (D >= 128) {
-    return rel_modes_qw<T, D, 16>(prm, stream);
+    return rel_modes_qw<T, D, 16>(prm, cus, stream);
   } else if constexpr (D == 32 && sizeof(T) == 2) {
-    if (prm.qw == 16 && prm.splits <= 1) return rel_modes_qw<T, D, 16>(prm, stream);
-    return rel_modes_qw<T, D, 32>(prm, stream);
+    if (prm.qw == 16 && prm.splits <= 1) return rel_modes_qw<T, D, 16>(prm, cus, stream);
+    return rel_modes_qw<T, D, 32>(prm, cus, stream);
   } else {
-    return rel_modes_qw<T, D, 32>(prm, stream);
+    return rel_modes_qw<T, D, 32>(prm, cus, stream);
   }
 }
 
@@ -2084,9 +2071,9 @@ size_t rel_attention_workspace_bytes(int splits, int B, int H, int L, int D) {
   return static_cast<size_t>(splits) * B * L * H * static_cast<size_t>(D + 2) * sizeof(float);
 }
 
-int launch_rel_attention(const RelParams& prm, int D, int dtype, hipStream_t stream) {
+int launch_rel_attention(const RelParams& prm, int D, int dtype, int cus, hipStream_t stream) {
 #define DFLASH_REL_CASE(TYPE, DIM) \
-  if (D == DIM) return rel_modes<TYPE, DIM>(prm, stream);
+  if (D == DIM) return rel_modes<TYPE, DIM>(prm, cus, stream);
   if (dtype == DFLASH_DTYPE_FP16) {
     DFLASH_REL_CASE(_Float16, 32) DFLASH_REL_CASE(_Float16, 64) DFLASH_REL_CASE(_Float16, 128)
   } else if (dtype == DFLASH_DTYPE_BF16) {
