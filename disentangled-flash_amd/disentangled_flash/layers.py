@@ -88,13 +88,26 @@ def _layernorm_fake(x, weight, bias, eps):
 USE_HIP_GEMM = True
 
 # Which GEMM runs an encoder projection (projection_on_hip): the hand-written one where
-# it fits (gemm_fits).  Device times from HIP graphs over changing operands, hand-written /
-# hipBLASLt (+ its GELU pass, + the fused add + LayerNorm for the output blocks), fp16, us:
-#   * width 768, 16384 rows: QKV 64.7 / 71.3, attention output 22.1 / 25.0, FFN
-#     intermediate + GELU 90 / 117, FFN output 77 / 71; 4096 rows: 18.1 / 19.7, 16.2 /
-#     18.2, 24.5 / 37.6, 29.7 / 30.3; 512 rows: 7.5 / 8.7, 9.2 / 11.2, 8.8 / 13.6, 13.6 /
-#     15.9; 64 rows: 5.4 / 7.6, 7.2 / 9.2, 5.6 / 10.5, 8.9 / 11.1;
-#   * an F.linear call also costs about 19 us of hipBLASLt host time against a few.
+# it fits (gemm_fits), but the FFN output (K = 4 x hidden) from LIBRARY_FFN_OUTPUT_MIN_ROWS
+# rows on hipBLASLt, which is faster there (output_on_hip).  Device times from HIP graphs
+# over changing operands, hand-written / hipBLASLt (+ its GELU pass, + the fused
+# add + LayerNorm for the output blocks), fp16, us, rows: QKV, attention output, FFN
+# intermediate + GELU, FFN output:
+#   width 768    512:   7.5 / 8.6,    9.0 / 9.7,    9.2 / 13.9,  14.0 / 16.3
+#               4096:  19.5 / 20.4,  15.6 / 18.8,  24.8 / 38.6,  33.3 / 33.0
+#               8192:  33.2 / 40.2,  23.0 / 25.4,  51.4 / 72.6,  50.2 / 49.9
+#              12288:  51.5 / 45.8,  30.3 / 39.0,  78.2 / 99.4,  85.2 / 74.8
+#              16384:  71.7 / 71.3,  37.5 / 38.7, 102.6 / 120.8, 91.3 / 84.7
+#   width 1024  4096:  27.3 / 30.6,  20.0 / 22.3,  38.5 / 50.2,  46.6 / 46.2
+#               8192:  54.0 / 59.6,  31.7 / 33.9,  75.7 / 91.4,  90.3 / 78.7
+#              16384: 104.1 / 88.4,  52.3 / 52.4, 156.7 / 175.9, 129.7 / 121.2
+#   width 1536  2048:  32.6 / 31.9,  22.3 / 23.7,  39.6 / 53.8,  55.7 / 52.6
+#               4096:  57.4 / 71.6,  31.8 / 33.3,  79.3 / 98.8,  85.1 / 85.3
+#               8192: 114.5 / 114.0, 50.9 / 53.1, 154.2 / 169.7, 151.7 / 139.6
+# An F.linear call also costs about 19 us of hipBLASLt host time against a few.  (The QKV
+# projection is behind in places too, by up to 20 %: its tiles leave a last round half
+# empty.)
+LIBRARY_FFN_OUTPUT_MIN_ROWS = 8192
 # torch.compile traces hip_gemm_rows's rule instead: below HIP_GEMM_MIN_ROWS rows F.linear,
 # which Inductor fuses.  Checked on every call: the layer program binds the fused steps once
 # per bucket, while B varies per call.
@@ -164,6 +177,16 @@ def projection_on_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor 
     # to look at, and the op's dispatch decides.)
     return not _lib.runs_directly(weight) \
         or (weight.data_ptr() % 16 == 0 and bias.data_ptr() % 8 == 0)
+
+
+def output_on_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
+    """:func:`projection_on_hip` for the projection of an output block, whose FFN form (``K``
+    at least twice ``N``) of many rows stays on ``F.linear``."""
+
+    n, k = weight.shape
+    if k >= 2 * n and k > 0 and x.numel() // k >= LIBRARY_FFN_OUTPUT_MIN_ROWS:
+        return False
+    return projection_on_hip(x, weight, bias)
 
 
 # Tile configuration the encoder asks dflash_linear_fwd for (bits 8.. of its
@@ -390,7 +413,7 @@ def output_block(module: nn.Module, hidden_states: torch.Tensor,
     residual = gemm_rows(input_tensor)
     norm = module.LayerNorm
     weight, bias = dense.weight, dense.bias
-    if isinstance(dense, nn.Linear) and projection_on_hip(hidden_states, weight, bias):
+    if isinstance(dense, nn.Linear) and output_on_hip(hidden_states, weight, bias):
         return linear_add_layernorm(gemm_rows(hidden_states), weight, bias, residual,
                                     norm.weight, norm.bias, norm.eps)
     projected = F.linear(hidden_states, weight, bias)
