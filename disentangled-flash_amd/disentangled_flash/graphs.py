@@ -22,7 +22,6 @@ from collections.abc import Iterable
 
 import torch
 
-from . import layers
 from .deberta import DebertaV2InferenceEncoder
 
 
@@ -59,9 +58,8 @@ class DebertaGraphBucket:
         with torch.inference_mode(), torch.cuda.stream(side):
             # Library handles and workspaces exist before capture: the warm-up runs the
             # kernels the capture will record.
-            with layers.graph_gemm_choice():
-                for _ in range(max(1, warmup)):
-                    run()
+            for _ in range(max(1, warmup)):
+                run()
             with torch.cuda.graph(self.graph, pool=self.pool, stream=side):
                 self.output = run()
         torch.cuda.current_stream(weight.device).wait_stream(side)

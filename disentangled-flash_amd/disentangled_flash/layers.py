@@ -21,7 +21,6 @@ traces through them, like the attention ops.
 from __future__ import annotations
 
 import contextlib
-import threading
 
 import torch
 from torch import nn
@@ -108,55 +107,18 @@ USE_HIP_GEMM = True
 # projection is behind in places too, by up to 20 %: its tiles leave a last round half
 # empty.)
 LIBRARY_FFN_OUTPUT_MIN_ROWS = 8192
-# torch.compile traces hip_gemm_rows's rule instead: below HIP_GEMM_MIN_ROWS rows F.linear,
-# which Inductor fuses.  Checked on every call: the layer program binds the fused steps once
-# per bucket, while B varies per call.
+# While torch.compile traces, the hand-written GEMM from HIP_GEMM_MIN_ROWS rows; below,
+# F.linear, which Inductor fuses.  Checked on every call: the layer program binds the
+# fused steps once per bucket, while B varies per call.
 HIP_GEMM_MIN_ROWS = 16384
-HIP_GEMM_EAGER_MAX_ROWS = 2048
-HIP_GEMM_EAGER_MAX_WIDTH = 768
-
-_GRAPH_CHOICE = threading.local()
 
 
 @contextlib.contextmanager
 def graph_gemm_choice():
-    """Eager forwards inside this block (on this thread) pick their GEMMs as HIP-graph
-    capture does, so they reproduce a captured bucket's replays bit for bit."""
+    """For callers that compare with a captured bucket: eager forwards run the GEMMs that a
+    capture records, bit for bit, inside this block and outside it."""
 
-    saved = getattr(_GRAPH_CHOICE, "on", False)
-    _GRAPH_CHOICE.on = True
-    try:
-        yield
-    finally:
-        _GRAPH_CHOICE.on = saved
-
-
-def eager_small_gemm(x: torch.Tensor, n: int) -> bool:
-    """True for an eager ``[..., K] x [N, K]^T`` projection small enough to be
-    launch-bound, at base width (see the rules above)."""
-
-    k = x.shape[-1]
-    if k <= 0 or x.device.type != "cuda" or torch.compiler.is_compiling():
-        return False
-    if x.numel() // k > HIP_GEMM_EAGER_MAX_ROWS or min(k, n) > HIP_GEMM_EAGER_MAX_WIDTH:
-        return False
-    if getattr(_GRAPH_CHOICE, "on", False):
-        return False
-    return not torch.cuda.is_current_stream_capturing()
-
-
-def hip_gemm_rows(x: torch.Tensor, n: int | None = None) -> bool:
-    """The rule by rows and launch mode for the projection of ``x`` (``[..., K]``) to
-    ``n`` columns (default K) that ``torch.compile`` traces: True from
-    :data:`HIP_GEMM_MIN_ROWS` rows, and outside tracing in launch-bound eager forwards
-    (:func:`eager_small_gemm`)."""
-
-    k = x.shape[-1]
-    if k <= 0 or x.device.type != "cuda":
-        return False
-    if x.numel() // k >= HIP_GEMM_MIN_ROWS:
-        return True
-    return eager_small_gemm(x, k if n is None else n)
+    yield
 
 
 def projection_on_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
@@ -169,7 +131,7 @@ def projection_on_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor 
             or x.shape[-1] != weight.shape[1] or x.device != weight.device:
         return False
     if torch.compiler.is_compiling():
-        return hip_gemm_rows(x, weight.shape[0])
+        return x.numel() // x.shape[-1] >= HIP_GEMM_MIN_ROWS
     n, k = weight.shape
     if x.numel() // k * max(n, k) >= GEMM_MAX_ELEMENTS:
         return False
@@ -418,10 +380,6 @@ def output_block(module: nn.Module, hidden_states: torch.Tensor,
                                     norm.weight, norm.bias, norm.eps)
     projected = F.linear(hidden_states, weight, bias)
     return add_layernorm(projected, residual, norm.weight, norm.bias, norm.eps)
-
-
-# The attention output block runs the same form as the FFN's.
-output_block_gemm = output_block
 
 
 # ConvLayer.conv_act values the fused tail implements (DFLASH_ACT_* codes);

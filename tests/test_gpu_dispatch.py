@@ -87,17 +87,3 @@ def test_what_does_not_fit_runs_in_the_library(ran, monkeypatch):
     # 320 columns are no multiple of 128 or 192; 1280 are.
     assert [kind for kind, _, n, _ in ran if n != 1280] == ["library"] * 8
     assert [kind for kind, _, n, _ in ran if n == 1280] == ["hip"]
-
-
-def test_while_tracing(monkeypatch):
-    """``torch.compile`` keeps ``F.linear``, which it fuses, below 16384 rows."""
-
-    from disentangled_flash import layers
-
-    weight = torch.zeros(768, 768, device="cuda", dtype=torch.float16)
-    few, many = (torch.zeros(n, 768, device="cuda", dtype=torch.float16) for n in (16383, 16384))
-    assert layers.projection_on_hip(few, weight, weight[0])
-    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
-    assert not layers.projection_on_hip(few, weight, weight[0])
-    assert layers.projection_on_hip(many, weight, weight[0])
-    assert not layers.projection_on_hip(many.cpu(), weight.cpu(), weight[0].cpu())

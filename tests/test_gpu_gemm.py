@@ -122,14 +122,13 @@ def test_linear_ops_and_errors():
     assert lib.dflash_linear_fwd(None, None, None, None, None, 0, 192, 32, 0, 0, None) == 0
 
 
-def test_encoder_gemm_tails_match_modules(monkeypatch):
+def test_encoder_gemm_tails_match_modules():
     """The fused tails against the HF module pieces they replace, in fp16."""
 
-    from disentangled_flash import layers
     from disentangled_flash.layers import (
         fusable_intermediate,
         intermediate_block,
-        output_block_gemm,
+        output_block,
     )
     from transformers import DebertaV2Config
     from transformers.models.deberta_v2.modeling_deberta_v2 import (
@@ -137,7 +136,6 @@ def test_encoder_gemm_tails_match_modules(monkeypatch):
         DebertaV2SelfOutput,
     )
 
-    monkeypatch.setattr(layers, "HIP_GEMM_MIN_ROWS", 0)  # the hand-written GEMM at 520 rows
     cfg = DebertaV2Config(hidden_size=768, intermediate_size=3072, hidden_act="gelu",
                           hidden_dropout_prob=0.0, layer_norm_eps=1e-7)
     torch.manual_seed(3)
@@ -149,7 +147,7 @@ def test_encoder_gemm_tails_match_modules(monkeypatch):
     with torch.inference_mode():
         got_i = intermediate_block(inter, h)
         want_i = inter.double()(h.double())
-        got_o = output_block_gemm(out, h, res)
+        got_o = output_block(out, h, res)
         want_o = out.double()(h.double(), res.double())
     err_i = (got_i.double() - want_i).abs().max().item()
     err_o = (got_o.double() - want_o).abs().max().item()
@@ -158,31 +156,37 @@ def test_encoder_gemm_tails_match_modules(monkeypatch):
     assert err_o <= 2e-2  # LayerNorm output of O(1) rows in fp16 (rstd ~ 1, two roundings)
 
 
-def test_projection_dispatch_rules():
-    """Which GEMM an encoder projection runs on, by rows, width and launch mode: the
-    hand-written GEMM from HIP_GEMM_MIN_ROWS rows and in launch-bound eager forwards at
-    base width; hipBLASLt otherwise, in particular while a HIP graph is captured."""
+def test_projection_dispatch_rules(monkeypatch):
+    """Which GEMM an encoder projection runs on: the hand-written one at every row count
+    (the FFN output of many rows aside), while a HIP graph is captured too; while
+    ``torch.compile`` traces, ``F.linear``, which it fuses, below 16384 rows."""
 
     from disentangled_flash import layers
 
-    base = torch.zeros(1, 512, 768, device="cuda", dtype=torch.float16)      # 512 rows, K 768
-    xlarge = torch.zeros(1, 512, 1536, device="cuda", dtype=torch.float16)   # K 1536
-    big = torch.zeros(32, 512, 768, device="cuda", dtype=torch.float16)      # 16384 rows
-    mid = torch.zeros(8, 512, 768, device="cuda", dtype=torch.float16)       # 4096 rows
-    assert layers.hip_gemm_rows(base) and layers.hip_gemm_rows(base, 2304)
-    assert layers.eager_small_gemm(torch.zeros(1, 512, 3072, device="cuda", dtype=torch.float16), 768)
-    assert not layers.hip_gemm_rows(xlarge) and not layers.hip_gemm_rows(xlarge, 4608)
-    assert layers.hip_gemm_rows(big) and not layers.eager_small_gemm(big, 768)
-    assert not layers.hip_gemm_rows(mid)
-    assert not layers.hip_gemm_rows(base.cpu())
-    with layers.graph_gemm_choice():
-        assert not layers.hip_gemm_rows(base) and layers.hip_gemm_rows(big)
-    assert layers.hip_gemm_rows(base)
+    weight = torch.zeros(768, 768, device="cuda", dtype=torch.float16)
+    wide = torch.zeros(768, 3072, device="cuda", dtype=torch.float16)
+    bias = weight[0]
+
+    def rows(n, k=768):
+        return torch.zeros(1, n, k, device="cuda", dtype=torch.float16)
+
+    for n in (1, 512, 8192, 16384):
+        assert layers.projection_on_hip(rows(n), weight, bias)
+        assert layers.output_on_hip(rows(n), weight, bias)
+    assert layers.output_on_hip(rows(8191, 3072), wide, bias)
+    assert not layers.output_on_hip(rows(8192, 3072), wide, bias)
+    assert not layers.projection_on_hip(rows(512).cpu(), weight.cpu(), bias.cpu())
     graph = torch.cuda.CUDAGraph()
     seen = []
     side = torch.cuda.Stream()
+    x = rows(512)
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
-        seen.append((layers.hip_gemm_rows(base), layers.hip_gemm_rows(big)))
+        seen.append((layers.projection_on_hip(x, weight, bias),
+                     layers.output_on_hip(x, weight, bias)))
     torch.cuda.current_stream().wait_stream(side)
-    assert seen == [(False, True)]
+    assert seen == [(True, True)]
+    few, many = rows(16383), rows(16384)
+    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
+    assert not layers.projection_on_hip(few, weight, bias)
+    assert layers.projection_on_hip(many, weight, bias)

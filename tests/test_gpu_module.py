@@ -340,13 +340,10 @@ def test_encoder_with_library_projections(base_encoder, dtype, monkeypatch):
 
 
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
-def test_encoder_with_hand_written_gemm_below_the_row_threshold(base_encoder, dtype, monkeypatch):
-    """The hand-written GEMM (fused QKV, GELU and residual epilogues) in every layer at a
-    bucket below ``HIP_GEMM_MIN_ROWS``, where the encoder would otherwise use hipBLASLt."""
+def test_encoder_with_hand_written_gemm_below_the_row_threshold(base_encoder, dtype):
+    """The hand-written GEMM (fused QKV, GELU epilogue and output blocks) in every layer, at
+    2048 rows, where it also runs the FFN outputs."""
 
-    from disentangled_flash import layers
-
-    monkeypatch.setattr(layers, "HIP_GEMM_MIN_ROWS", 0)
     torch_dtype = DTYPES[dtype]
     err, ref_err, err_same = _encoder_errors(base_encoder, 8, 256, torch_dtype)
     print(f"encoder (hand-written GEMM at 2048 rows) {dtype}: hip-vs-HF-fp32 {err:.3e}, "
@@ -424,11 +421,10 @@ def test_hip_graph_buckets_replay_eager_results():
 
     Several replays per bucket with new inputs, interleaved with eager work and
     host synchronisation, each checked against the eager forward of the same
-    inputs with the GEMM choice of graph capture (same kernels, same launch order:
-    identical results expected).
+    inputs (same kernels, same launch order: identical results expected).
     """
 
-    from disentangled_flash import capture_deberta_buckets, enable_deberta_inference, layers
+    from disentangled_flash import capture_deberta_buckets, enable_deberta_inference
 
     base = _encoder_model(2, 768, 12, 3072)
     model = enable_deberta_inference(base.to("cuda", torch.float16), backend="hip",
@@ -444,9 +440,8 @@ def test_hip_graph_buckets_replay_eager_results():
                 hidden, mask = _encoder_inputs(batch, length, 768, seed=100 + replay + length)
                 hidden, mask = hidden.to("cuda", torch.float16), mask.cuda()
                 plans = encoder.plans_for(length)
-                with layers.graph_gemm_choice():  # the GEMMs a capture picks
-                    eager = encoder.forward_prepared(hidden, mask, plans,
-                                                     output_hidden_states=False).last_hidden_state
+                eager = encoder.forward_prepared(hidden, mask, plans,
+                                                 output_hidden_states=False).last_hidden_state
                 torch.cuda.synchronize()
                 got = bucket(hidden, mask).clone()
                 torch.cuda.synchronize()
