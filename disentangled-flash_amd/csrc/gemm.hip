@@ -131,9 +131,10 @@ __device__ inline float gelu_erf(float x) {
 
 // One buffer_load_dwordx4 with the LDS bit: 16 bytes per lane from `off` + `scalar`
 // (`scalar` uniform; zeros where `off` is past the resource's size) to LDS at `lds` + 16 *
-// lane (`lds` uniform, in M0; one wait state between the write of M0 and the load).  Inline
-// assembly, so that the compiler does not wait for copies in flight before fragment reads;
-// they are awaited by wait_vmem and the slab's barrier.
+// lane (`lds` uniform, in M0, which nothing else in these kernels uses and clang does not take
+// as a clobber; one wait state between the write of M0 and the load).  Inline assembly, so
+// that the compiler does not wait for copies in flight before fragment reads; they are
+// awaited by wait_vmem and the slab's barrier.
 __device__ inline void copy16_to_lds(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t scalar,
                                      uint32_t lds) {
   asm volatile(

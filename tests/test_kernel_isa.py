@@ -30,19 +30,23 @@ COPY = re.compile(r"^\s+buffer_load_dwordx4\s.*\blds\b")
 EXPLICIT_WAIT = re.compile(r"^\s+s_waitcnt vmcnt\((\d+)\)\s*$")
 
 
-@pytest.fixture(scope="module")
-def attention_asm(tmp_path_factory):
+def _assembly(directory: Path, source: str) -> str:
     sys.path.insert(0, str(CSRC))
     import build  # noqa: E402
 
     if shutil.which("hipcc") is None and not Path("/opt/rocm/bin/hipcc").exists():
         pytest.skip("hipcc not available")
-    out = tmp_path_factory.mktemp("isa") / "rel_attention.s"
+    out = directory / "kernels.s"
     cmd = [build.hipcc(), *build.COMMON_FLAGS, "-I", str(CSRC), "--offload-device-only", "-S",
-           str(CSRC / "rel_attention.hip"), "-o", str(out)]
+           str(CSRC / source), "-o", str(out)]
     result = subprocess.run(cmd, capture_output=True, text=True)
     assert result.returncode == 0, result.stderr[-2000:]
     return out.read_text()
+
+
+@pytest.fixture(scope="module")
+def attention_asm(tmp_path_factory):
+    return _assembly(tmp_path_factory.mktemp("isa"), "rel_attention.hip")
 
 
 def _kernels(asm: str):
@@ -116,3 +120,24 @@ def test_direct_copy_waits_cover_the_copies(attention_asm):
                 if VMEM.match(lines[j]) and not COPY.match(lines[j]):
                     count += 1
     assert checked > 0, "no kernel with direct copies was found"
+
+
+def test_gemm_copies_own_m0(tmp_path):
+    """The GEMM's copies set M0 in inline assembly without restoring it (M0 cannot be named as
+    clobbered): no other instruction of those kernels may use it."""
+
+    asm = _assembly(tmp_path, "gemm.hip")
+    names = re.findall(r"^(_ZN6dflash11gemm_kernel\w+):", asm, re.M)
+    assert names
+    copies = 0
+    for name in names:
+        start = asm.index(f"\n{name}:") + 1
+        inside = False
+        for line in asm[start:asm.index(".Lfunc_end", start)].splitlines():
+            if ";;#ASMSTART" in line or ";;#ASMEND" in line:
+                inside = ";;#ASMSTART" in line
+            elif inside:
+                copies += "lds" in line
+            else:
+                assert not re.search(r"\bm0\b", line.split(";")[0]), (name, line)
+    assert copies > 0
