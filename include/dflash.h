@@ -282,6 +282,9 @@ DFLASH_API int dflash_conv_layer_tail_fwd(const void* z, int z_dtype, const void
  *              slabs; 9 = 128 x 64, two per CU; 10 = 64 x 64, two per CU, five slabs;
  *              11 = 32 x 64, two per CU, six slabs.  A configuration whose columns do
  *              not divide N returns DFLASH_ERR_SHAPE.
+ * Sums are fp32.  Their order depends on M and on the tile that a row lies in: repeated
+ * calls give the same bits, but a row can differ in its last bits at another place of
+ * the batch or in a batch of another size.
  */
 DFLASH_API int dflash_linear_fwd(const void* x, const void* weight, const void* bias,
                                  const void* residual, void* y, int M, int N, int K,

@@ -93,3 +93,37 @@ def test_rows_past_32_bit_offsets():
         # times that allowed.
         _, excess = _check(y, ref, lin, acc + 10 * 2.0 ** -15, torch.float16, 2)
         assert excess <= 0, (config, excess)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("config", [0, 2, 6, 10])
+def test_equal_rows(dtype, config):
+    """A row's fp32 sums run in an order that depends on its tile: equal rows agree to the
+    bound of any order (half a unit of the type each, and the fp32 sums), repeated calls to
+    the bit."""
+
+    m, k, n = 2048, 1536, 256
+    x, w, b, r = _inputs(1, k, n, dtype, seed=11)
+    x, r = x.expand(m, k).contiguous(), r.expand(m, n).contiguous()
+    ref, lin, acc = _reference(x, w, b, r, 0, dtype)
+    first = None
+    for _ in range(3):
+        code, y = _run(x, w, b, None, 0, config)
+        assert code == 0
+        assert first is None or torch.equal(y, first)
+        first = y
+    _, excess = _check(first, ref, lin, acc, dtype, 0)
+    assert excess <= 0
+
+
+@pytest.mark.parametrize("epilogue", [0, 1])
+@pytest.mark.parametrize("m", [8191, 8200])
+def test_outputs_around_64_mib(m, epilogue):
+    """Outputs below and above the size where plain ones are no longer written through the L2."""
+
+    x, w, b, r = _inputs(m, 96, 4096, torch.bfloat16, seed=m)
+    ref, lin, acc = _reference(x, w, b, r, epilogue, torch.bfloat16)
+    code, y = _run(x, w, b, None, epilogue)
+    assert code == 0
+    _, excess = _check(y, ref, lin, acc, torch.bfloat16, epilogue)
+    assert excess <= 0
