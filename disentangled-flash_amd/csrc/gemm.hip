@@ -453,11 +453,15 @@ int launch_copies(GemmArgs args, hipStream_t stream) {
   if (err != hipSuccess) return static_cast<int>(err);
   args.m_blocks = (args.M + CF::BM - 1) / CF::BM;
   args.n_blocks = args.N / CF::BN;
-  // Y through the L2 unless it is large: 12 layers of 4096 rows, 768 wide (Y of 6 to 25 MB)
-  // 1416 us, left in the L2 1462, non-temporal 1508; one layer of 16384 rows, with QKV
-  // and FFN outputs of 75 and 100 MB, 357, 349 and 363 us.
+  // Y through the L2 (against left in it: 12 layers of 4096 rows, 768 wide, Y of 6 to 24 MiB,
+  // 1416 us against 1462, non-temporal 1508), except a plain output of 64 MiB and more: the
+  // QKV output of one ragged 768-wide layer at 12288 rows (54 MiB) even, at 16384 (72
+  // MiB) 2.3 % slower through it, as the attention reads it at once.  The FFN intermediate
+  // gains at every size, us, left / through: 8192 rows (48 MiB) 214.1 / 207.5, 12288 (72
+  // MiB) 316.0 / 305.1, 16384 (96 MiB) 380.2 / 370.5.
   args.through = args.N <= kMaxThroughN &&
-                 static_cast<int64_t>(args.M) * args.N * 2 < (int64_t{48} << 20);
+                 (EPI == kEpiBiasGelu ||
+                  static_cast<int64_t>(args.M) * args.N * 2 < (int64_t{64} << 20));
   // XCDs along the rows and the columns: the split with the fewest rows of X and W
   // for an XCD to read, among those whose largest range needs no more tiles than an
   // even share rounded up to whole rounds of its CUs.
