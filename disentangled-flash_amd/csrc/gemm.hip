@@ -14,22 +14,22 @@
 //                  of DebertaV2SelfOutput / DebertaV2Output before LayerNorm,
 //                  _reference.py:108-112, 482-485)
 //
-// What bounds it.  With tiles of 256 rows the k-loop is near the matrix unit:
-// at M = 16384, N = K = 3072 (fp16) the 256 x 256 tile takes 235 us, 1.32
-// PFLOP/s, its matrix pipe busy 66-70 % at the clock the power limit leaves
-// (1.8 GHz); a loop of 32-deep steps in the compiler's own order took 292 us.  At
-// K = 768 the rest is the start of a tile and the stores at its end (16384 rows:
-// QKV 62 us, 920 TFLOP/s; FFN intermediate with GELU 85-90 us); with few rows it is the
-// latency of the copies.
+// What bounds it.  With tiles of 256 rows and a long K the loop is near the matrix unit:
+// at M = 16384, N = K = 3072 (fp16) the 256 x 256 tile takes 232-254 us (two chips), 1.2-1.3
+// PFLOP/s, its matrix pipe busy 67-69 % at the clock the power limit leaves
+// (1.8 GHz); a loop of 32-deep steps in the compiler's own order took 292 us against 235.  At
+// K = 768 the start of a tile and the stores at its end are as long as the loop (16384 rows:
+// QKV 62-73 us, pipe busy 42 %; FFN intermediate with GELU 88-93 us, 39 %); with few rows it is
+// the latency of the copies.  (profiles/gemm_sq_counters.md)
 
 // Slabs of 64 k.  X and W are copied straight into LDS (buffer loads with the
 // LDS bit, 16 bytes a lane: no registers, no address arithmetic in the loop)
 // as slabs of 64 k, so that a row of a copy is one whole 128-byte line: with
 // 32-deep slabs (64-byte rows) L2 serves twice as many requests for the same
 // bytes (256 x 256 tile, N = K = 3072: 250 against 235 us).  A slab row is 128 bytes of LDS whose
-// eight 16-byte chunks are permuted by slab_swizzle(row), which makes the
-// MFMA fragment reads (16 rows x one chunk per 16 lanes) conflict-free.  STAGES
-// slabs form a ring.
+// eight 16-byte chunks are permuted by slab_swizzle(row), so that of the 16 rows
+// whose chunk 16 lanes read (an MFMA fragment) no two lie in the same banks; the counters still
+// show four conflict cycles a read.  STAGES slabs form a ring.
 //
 // One slab is two 32-deep MFMA steps.  The fragments of a step are read from
 // LDS during the MFMAs of the step before (two register sets).  Between the

@@ -737,9 +737,10 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
   TW tcv[TC_N];
   TW tpv[TP_N];
   // A lane reads rows r0 + m TC_R of one lookup's slot.  The range check of a
-  // raw buffer covers voffset (and the instruction offset) but not soffset.
+  // raw buffer is documented to cover voffset (and the instruction offset) but
+  // not soffset (the MI355X was seen to compare the sum; not relied on).
   // The fast form puts the row step in soffset (one address register per
-  // lookup); a row past L then reads outside the (b, h) slice - inside the
+  // lookup); a row past L then may read outside the (b, h) slice - inside the
   // tensor for every slice but the last, whose query blocks and key tiles
   // therefore run the ROWSAFE instance when L is not a multiple of the tile
   // (see launch_rel).  ROWSAFE carries the whole offset in voffset, so rows
@@ -762,7 +763,7 @@ __global__ __launch_bounds__(kThreads, WGS) void rel_attention_kernel(RelParams 
   // Slots of the windows of the tile at key offset j0.  A lookup entry
   // outside [0, S) is clamped to S - 1: its value is undefined (as in the
   // reference), but its offset stays inside its table row, so that with the
-  // row step in soffset (unchecked) no read leaves the tensor.
+  // row step in soffset no read leaves the tensor by either rule.
   const uint32_t slot_max = static_cast<uint32_t>(p.S - 1);
   auto table_lookups = [&](int j0, auto sel) {
     if constexpr (TC && (decltype(sel)::value & 1)) {

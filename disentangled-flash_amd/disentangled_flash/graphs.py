@@ -1,9 +1,8 @@
 """HIP-graph buckets: replay a prepared encoder forward without host launch cost.
 
-At small batches the eager encoder is bound by the host, not the GPU: each
-layer issues its projections, the attention and the LayerNorms from Python, so a
-12-layer forward costs about a millisecond of host time whatever the batch.  A HIP graph
-records the whole launch sequence of one (batch, bucket length) once and
+At small batches an eager forward is bound by its launches: even as one library call a
+layer (``native.py``) it issues about 84, and the program's own host work comes on top.
+A HIP graph records the whole launch sequence of one (batch, bucket length) once and
 replays it with a single host call.
 
 This is the MI355X-side counterpart of ``compile_deberta_buckets`` (reference

@@ -2,10 +2,11 @@
 
 ``DebertaV2SelfOutput`` and ``DebertaV2Output`` (reference ``_reference.py:101-112``
 and ``474-485``) both end in ``LayerNorm(dense(x) + input_tensor)``.  The HIP
-encoder runs the dense projection on the hand-written GEMM (:func:`linear_epilogue`)
-where :func:`projection_on_hip` says so, on ``F.linear`` otherwise, and replaces the
-separate residual add and LayerNorm with one kernel, ``disentangled_flash::add_layernorm``, which reads the projection and
-the residual once and writes the normalised row.
+encoder runs the dense projection on the hand-written GEMM where
+:func:`projection_on_hip` and :func:`output_on_hip` say so
+(``disentangled_flash::linear_add_layernorm``), on ``F.linear`` otherwise, and replaces the
+separate residual add and LayerNorm with one kernel (``disentangled_flash::add_layernorm``),
+which reads the projection and the residual once and writes the normalised row.
 
 The ``ConvLayer`` run after the first encoder layer (reference
 ``_reference.py:519-566``, called at ``deberta.py:272-273``) is fused the same
@@ -83,7 +84,7 @@ def _layernorm_fake(x, weight, bias, eps):
 
 # Whether the encoder runs its projections on the hand-written GEMM
 # (dflash_linear_fwd) where it fits, or on hipBLASLt through F.linear; read when
-# an encoder is prepared and on every QKV projection.  A switch for A/B timing.
+# an encoder is prepared and on every projection.  A switch for A/B timing.
 USE_HIP_GEMM = True
 
 # Which GEMM runs an encoder projection (projection_on_hip): the hand-written one where
