@@ -501,13 +501,14 @@ int launch_gemm(const GemmArgs& args, hipStream_t stream) {
 //   rounds of CUs * WGS tiles, each fixed + slabs * slab time; the slab time of a
 //   round with n tiles is slab1 + slab1_load * n / CUs while every CU has at most
 //   one tile, and reaches slab_full with WGS tiles on a CU; gelu: the GELU epilogue.
-// The constants are a least-squares fit (in the logarithm) to 900 timings (HIP
-// graphs of back-to-back calls over weights and activations that change from call to
-// call, fp16): K and N of 768- and 1536-wide layers (all four projections),
-// M = 16 .. 16384, every configuration.  Taking the configuration with the smallest
-// modelled time is then 0.6 % slower on average than taking the fastest one of
-// each shape, and at most 13 %.  The CUs are those of the device; the constants are
-// an MI355X's.
+// The constants are a least-squares fit (in the logarithm) to timings of every
+// configuration at K and N of 768- and 1536-wide layers (all four projections) and M = 16 ..
+// 16384 (HIP graphs of back-to-back calls over weights and activations that change from call
+// to call, fp16).  bench.py --gemm-table times such a set: taking the configuration with the
+// smallest modelled time was 0.6-0.9 % slower on average than taking the fastest one of
+// each shape, and at most 12-14 % (80 shapes, two chips;
+// profiles/gemm_projection_device_times.md).  The CUs are those of the device; the
+// constants are an MI355X's.
 struct GemmCost {
   float fixed, slab1, slab1_load, slab_full, gelu;
 };
