@@ -300,25 +300,21 @@ def _is_erf_gelu(act) -> bool:
     return inner is F.gelu or getattr(inner, "__name__", "") == "_gelu_python"
 
 
-def _is_plain_call(module: nn.Module) -> bool:
-    """True if ``module(x)`` is its class's ``forward`` and nothing else: no forward hooks of
-    its own, no ``forward`` set on the instance."""
-
-    return not (module._forward_hooks or module._forward_pre_hooks
-                or "forward" in module.__dict__)
-
-
 def intermediate_is_dense_gelu(module: nn.Module) -> bool:
     """True if calling ``module`` (a :func:`fusable_intermediate` when the encoder was prepared)
-    still is its dense layer and an erf GELU: nothing was hooked, wrapped or replaced."""
+    still is its dense layer and an erf GELU: no forward hooks on any of the three or on all
+    modules, no ``forward`` set on an instance, nothing replaced."""
 
     modules = module._modules  # (past nn.Module's attribute lookup: this runs on every call)
     dense, act = modules.get("dense"), modules.get("intermediate_act_fn")
     if act is None:
         act = module.__dict__.get("intermediate_act_fn")
-    return isinstance(dense, nn.Linear) and _is_plain_call(module) and _is_plain_call(dense) \
-        and _is_erf_gelu(act) and (act is F.gelu or _is_plain_call(act)) \
-        and not (torch_module._global_forward_hooks or torch_module._global_forward_pre_hooks)
+    elif act._forward_hooks or act._forward_pre_hooks or "forward" in act.__dict__:
+        return False
+    return isinstance(dense, nn.Linear) and _is_erf_gelu(act) and not (
+        module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__
+        or dense._forward_hooks or dense._forward_pre_hooks or "forward" in dense.__dict__
+        or torch_module._global_forward_hooks or torch_module._global_forward_pre_hooks)
 
 
 def intermediate_block(module: nn.Module, hidden_states: torch.Tensor) -> torch.Tensor:

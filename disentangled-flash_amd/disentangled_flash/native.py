@@ -76,11 +76,11 @@ class NativeLayer:
         width = heads * dim
         inner_dense = self.intermediate._modules["dense"]
         inner = inner_dense.out_features
+        # (gemm_width_fits of the four projections: their K are multiples of 32 where the
+        # columns of the others fit and the head dimension is one of these.)
         if dim not in SUPPORTED_HEAD_DIMS or dtype not in layers.GEMM_DTYPES \
-                or not layers.gemm_width_fits(3 * width, hidden) \
-                or not layers.gemm_width_fits(hidden, width) \
-                or not layers.gemm_width_fits(inner, hidden) \
-                or not layers.gemm_width_fits(hidden, inner):
+                or (3 * width % 128 and 3 * width % 192) or (hidden % 128 and hidden % 192) \
+                or (inner % 128 and inner % 192):
             return None
         tail, last = self.attention_output._modules, self.output._modules
         attention_norm, output_norm = tail["LayerNorm"], last["LayerNorm"]
